@@ -1,0 +1,84 @@
+"""The single launch's batch units (k_layer_batch) against the stream-ordered kernels, whose decode
+units compute the same sums: bit for bit at chunk sizes around the units' tiles (32, 64 and 128
+rows and their remainders, more than one chunk an expert, experts no token picks), for both
+activation forms, with a shared expert of several chunks, K parts and the block steps; and
+against the CPU oracle once per form."""
+
+from __future__ import annotations
+
+from dataclasses import replace
+
+import pytest
+import torch
+
+from oracle import layer, metrics
+from vibe_megakernel_amd import cases as C
+from vibe_megakernel_amd import submission, workloads
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+MIXTRAL, DEEPSEEK, KIMI = "moe-fp8-mixtral-t16", "moe-fp8-deepseek-v3-t64", "moe-fp8-kimi-k2-t128"
+
+
+def _case(base, act="fp8", **p):
+    return replace(C.development(C.case(base), **p), activations=act)
+
+
+def _cases():
+    out = []
+    for act in ("fp8", "bf16"):
+        # Every token picks both experts: each holds `tokens` rows.
+        out += [_case(MIXTRAL, act, tokens=t, experts=2, topk=2) for t in (17, 32, 33, 64, 65, 96, 128, 129, 257)]
+        # Ragged rows per expert; one K block a row of h; an odd number of K blocks; rows of H = 4096
+        # (W8A8: gate and up apart, in both forms); K parts of the down units.
+        out.append(_case(MIXTRAL, act, tokens=200, experts=8, intermediate=128))
+        out.append(_case(MIXTRAL, act, tokens=300, experts=16, topk=3, hidden=768, intermediate=384))
+        out.append(_case(MIXTRAL, act, tokens=70, experts=8, hidden=4096, intermediate=512))
+        out.append(_case(DEEPSEEK, act, tokens=261))
+        out.append(replace(_case(DEEPSEEK, act, tokens=300, shared_experts=2), norm="fp32_weight", residual=True))
+        out.append(_case(KIMI, act, tokens=500, experts=32, topk=2))  # skewed: most experts hold few rows, some none
+    out.append(replace(_case(DEEPSEEK, tokens=270), swiglu="bf16", swiglu_limit=0.5, power_of_two=True))
+    return out
+
+
+def _id(c):
+    return f"{c.model.split('/')[-1].split()[0]}-{c.activations}-t{c.tokens}-e{c.experts}-h{c.hidden}-i{c.intermediate}"
+
+
+@pytest.mark.parametrize("case", _cases(), ids=_id)
+def test_batch_units_equal_the_stream_ordered_kernels(case):
+    print(_id(case), flush=True)
+    one, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
+    for seed in (3, 4):  # consecutive calls on one workspace
+        values = {k: v.to(DEV) for k, v in workloads.make_inputs(case, seed, "cpu").items()}
+        a, b = one(values), five(values)
+        torch.cuda.synchronize()
+        assert not one.gave_up(torch.device(DEV))
+        for k in ("y", "expert_ids", "expert_weights"):
+            assert torch.equal(a[k], b[k]), k
+
+
+def test_batch_kernel_runs_and_is_one_launch():
+    case = _case(DEEPSEEK, tokens=256)
+    run = submission.MoELayer(case)
+    values = {k: v.to(DEV) for k, v in workloads.make_inputs(case, 3, "cpu").items()}
+    run(values)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        run(values)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "k_" in e.name]
+    assert len(names) == 1 and "k_layer_batch" in names[0], names
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+def test_batch_units_against_the_oracle(act):
+    case = _case(MIXTRAL, act, tokens=150, experts=4)
+    values = workloads.make_inputs(case, 11, "cpu")
+    want = layer.reference(case, values)
+    got = submission.MoELayer(case)({k: v.to(DEV) for k, v in values.items()})
+    torch.cuda.synchronize()
+    assert torch.equal(got["expert_ids"].cpu(), want["expert_ids"])
+    check = metrics.layer_checks(got["y"], want["y"])  # the layer's bars: max-rel 1e-2, cosine 0.9999
+    assert check["pass"], check

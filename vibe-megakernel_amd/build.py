@@ -26,6 +26,10 @@ FLAGS = [
     "-ffp-contract=off",
     # No packed fp32 VALU instructions.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # MFMA results in vector registers, also in kernels planned for one wavefront per SIMD: the
+    # fp8 units scale every result by fp32 block scales, and a result in an accumulation register
+    # costs a copy per element first.
+    "-mllvm", "-amdgpu-mfma-vgpr-form",
     # Per-kernel register, spill and scratch figures (remarks on stderr).
     "-Rpass-analysis=kernel-resource-usage",
 ]

@@ -1059,6 +1059,7 @@ constexpr int kMetaHit = 0, kMetaUnitsGU = 1, kMetaUnitsDN = 2, kMetaQueueGU = 3
               kMetaWide = 5, kMetaError = 32, kMetaInts = 64;
 constexpr int kChunkRows = 64;     // rows per chunk of the fp8 form (column tiles of up to 4)
 constexpr int kChunkRowsA16 = 32;  // of its W8A16 form (bf16 activations: column tiles of up to 2)
+constexpr int kChunkRowsBatch = 128;  // of the single launch's batch form
 constexpr int kChunkRowsMx = 128;  // of the MXFP4 form: wide units over 33-128 rows, narrow up to 32
 
 struct PermuteOut {
@@ -1513,6 +1514,16 @@ __device__ __forceinline__ i32x8 load_k32(const uint8_t* p) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// Calls f(std::integral_constant<int, I>{}) for I = B .. E-1 (a loop whose index is a
+// compile-time constant in the body).
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
 // Waits until at most N vector memory operations of this wavefront are outstanding.
 // The memory clobber keeps the compiler from moving loads across the wait.
 template <int N>
@@ -1809,12 +1820,11 @@ __device__ __forceinline__ void compute_stage(uint32_t slot, const LaneTile& lt,
 // first weights, which only makes the first stage's vmcnt wait below more conservative).
 //
 // The stream starts at K block `rot` and wraps around (any rot in [0, nkb); callers derive
-// it from the unit index). Units that run at the same time then read different K blocks of
+// it from the weight block, so a row's sum does not depend on the form of unit that takes it). Units that run at the same time then read different K blocks of
 // their weight rows: with every workgroup at the same K block, the addresses in flight
 // differ only in their high bits (multiples of the row length, 4 KiB for some models), and
 // the HBM channels serve them unevenly (about 6% slower on a Mixtral-shaped layer). The
-// fp32 sum over K blocks then runs in a rotated order; it depends on the work list only,
-// so results are still the same on every call.
+// fp32 sum over K blocks then runs in a rotated order, the same on every call.
 //
 // The wait for stage s: a wavefront's vector memory loads (to LDS or to registers)
 // complete in issue order, and the compiler's own counters do not cover the LDS that
@@ -1989,6 +1999,255 @@ struct ChunkRows {
   int out_base;  // (the dense schedule: expert e's rows e*T + t)
 };
 
+// The stream of the batch units (k_layer_batch, one workgroup per CU): 256 weight rows by up
+// to 128 activation rows, every operand through LDS. The four wavefronts move a stage together by
+// DMA, whole 128-byte lines (8 rows an instruction, XOR-swizzled 16-byte chunks), into one of 2-4
+// slots, a barrier per stage makes it visible, and wave w multiplies weight tiles 8*(w%2) .. +7
+// with activation tiles NT*(w/2) .. +NT-1 (128 rows by 16*NT columns).
+//
+// Why: a CU's vector L1 serves one 64-byte access a cycle and keeps a bounded number of bytes
+// pending, so what bounds a chunk of tens of rows is what passes through the L1. The decode units
+// load activations in the MFMA layout (16 rows by 16 bytes an instruction: 64 accesses for 1 KB,
+// line-wise 16), each wave for itself, and stream an expert's weights once per 64 rows.
+constexpr int kBatchRing = 147456;            // LDS bytes of the slots
+constexpr int kBatchWeights = 16 * kTileBytes;  // of a slot: 256 weight rows by 128 bytes
+constexpr int kBatchScales = 4 * 4 * 512;       // of the scales: per slot and wave 64 activation, 64 weight lanes
+
+// NT: 16-row activation tiles per wave, 2*NT of a chunk. A16 rows have 256 bytes a K block.
+template <int NT, bool A16>
+struct BatchStage {
+  static constexpr int kBytes = kBatchWeights + 2 * NT * kTileBytes * (A16 ? 2 : 1);
+  static constexpr int kSlots = kBatchRing / kBytes < 4 ? kBatchRing / kBytes : 4;
+  static constexpr int kLoads = NT * (A16 ? 2 : 1);  // activation DMA instructions per wave and stage
+  static_assert(kSlots >= 2 && (NT == 1 || NT == 2 || NT == 4), "slots of the batch ring");
+};
+
+template <int NT, bool A16>
+struct BatchOperands {
+  const uint8_t* a[4];  // row 0 of the four weight tiles this wave moves (tiles 4w .. 4w+3)
+  int lda;
+  const uint8_t* spare;  // as Operands::spare
+  const float* sw;      // weight scale row of this wave's tiles 0-3 (even lanes) and 4-7 (odd lanes)
+  const uint8_t* b[BatchStage<NT, A16>::kLoads];  // this lane's row and swizzled chunk of K block 0
+  const float* sx;      // the scale row of this wave's activation row l (mod 16*NT)
+};
+
+// This lane's activation row of its wave's DMA instruction i: instruction q = w*kLoads + i moves
+// the 8 rows 8q .. 8q+7 (W8A8), or of tile q / 4 the 8 rows of half q % 2 and the 128-byte half
+// q / 2 % 2 of the block's 256 (W8A16).
+template <int NT, bool A16, class F>
+__device__ __forceinline__ void batch_rows(BatchOperands<NT, A16>& o, const uint8_t* m, size_t ld, int n, F&& row) {
+  constexpr int L = BatchStage<NT, A16>::kLoads;
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane >> 3;
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int q = w * L + i, r = A16 ? 16 * (q >> 2) + 8 * (q & 1) + lr : 8 * q + lr;
+    o.b[i] = m + (size_t)row(min(r, n - 1)) * ld + (A16 ? ((q >> 1) & 1) * kBlock : 0) + (((lane & 7) ^ lr) << 4);
+  }
+}
+
+// LDS reads of the batch stream in inline asm (see read_slot), at compile-time offsets; lds_wait
+// waits until at most N are pending and names the results it covers, lds_arrived names more.
+template <int OFF>
+__device__ __forceinline__ void lds_read2(i32x4& a, i32x4& b, uint32_t pa, uint32_t pb) {
+  asm volatile("ds_read_b128 %0, %2 offset:%c4\n\tds_read_b128 %1, %3 offset:%c4"
+               : "=&v"(a), "=&v"(b)
+               : "v"(pa), "v"(pb), "i"(OFF)
+               : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void lds_read_f(float& v, uint32_t p) {
+  asm volatile("ds_read_b32 %0, %1 offset:%c2" : "=&v"(v) : "v"(p), "i"(OFF) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(i32x4& a, i32x4& b) {
+  asm volatile("s_waitcnt lgkmcnt(%c2)" : "+v"(a), "+v"(b) : "i"(N));
+}
+__device__ __forceinline__ void lds_arrived(i32x4& a, i32x4& b) { asm volatile("" : "+v"(a), "+v"(b)); }
+__device__ __forceinline__ void lds_arrived(float& a) { asm volatile("" : "+v"(a)); }
+
+// The weights of K block kb into a slot; past the last one (not live) as many loads from the spare
+// region, as issue_a.
+template <int NT, bool A16>
+__device__ __forceinline__ void issue_batch_weights(uint8_t* slot, const BatchOperands<NT, A16>& o, const LaneTile& lt,
+                                                    int w, int kb, bool live) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const uint8_t* base = live ? o.a[t] + (size_t)kb * kBlock : o.spare;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(base + (uint32_t)(lt.dma + 8 * i * o.lda)),
+          (__attribute__((address_space(3))) void*)(slot + (4 * w + t) * kTileBytes + i * 1024), 16, 0, kNonTemporal);
+  }
+}
+
+// The activations of K block kb, the weight scales and (W8A8) those of this wave's 16*NT
+// activation rows. The scales go through LDS as well: a register load among the LDS DMA would have
+// the compiler drain every load before its use.
+template <int NT, bool A16>
+__device__ __forceinline__ void issue_batch_acts(uint8_t* slot, uint8_t* scales, const BatchOperands<NT, A16>& o, int w,
+                                                 int kb) {
+  constexpr int L = BatchStage<NT, A16>::kLoads;
+#pragma unroll
+  for (int i = 0; i < L; ++i)
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void*)(o.b[i] + (size_t)kb * kBlock * (A16 ? 2 : 1)),
+        (__attribute__((address_space(3))) void*)(slot + kBatchWeights + (w * L + i) * 1024), 16, 0, 0);
+  if constexpr (!A16)
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(o.sx + kb),
+                                     (__attribute__((address_space(3))) void*)scales, 4, 0, 0);
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(o.sw + kb),
+                                   (__attribute__((address_space(3))) void*)(scales + 256), 4, 0, 0);
+}
+
+// Issue order: the weights of the first kSlots - 1 stages, (the wait,) their activations, then at
+// stage kb, after its barrier (every wave has read stage kb - 1), stage kb + kSlots - 1 into the
+// slot of kb - 1. When stage kb is waited for, the stages kb+1 .. kb+kSlots-2 were issued after it
+// (in the first round at least their activations): vmcnt <= (kSlots - 2) * their loads. Every
+// stage, live or not, issues the same loads and passes the same barrier; only the MFMAs of stages
+// past the end are skipped.
+//
+// The LDS reads are inline asm, waited for by count (they return in order; scalar loads in flight
+// only make the count larger): the activations and scales first, then two weight tiles at a time
+// under the MFMAs of the two before (one for 64 rows of bf16, whose activations fill the registers).
+template <int NT, bool A16>
+__device__ __forceinline__ void stream_gemm_batch(const BatchOperands<NT, A16>& op, int nkb, int rot, uint8_t* ring,
+                                                  f32x4 (&acc)[8][NT], const ReadyWait& ready) {
+  using St = BatchStage<NT, A16>;
+  constexpr int W = A16 && NT == 4 ? 1 : 2;  // weight tiles per group of LDS reads (registers)
+  constexpr int D = St::kSlots, kChunks = A16 ? 4 : 2, kAct = St::kLoads + (A16 ? 1 : 2);
+  auto phys = [nkb, rot](int kb) {
+    const int p = min(kb, nkb - 1) + rot;
+    return p >= nkb ? p - nkb : p;
+  };
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = w & 1, wn = w >> 1;
+  const LaneTile lt = lane_tile(op.lda);
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring;
+  uint8_t* const scales = ring + kBatchRing + w * 512;  // + 2048 per slot
+  // This lane's chunks of a 16-row activation tile: g and g + 4 of its 128-byte row (W8A8); 2g and
+  // 2g + 1 of each 128-byte half (W8A16, whose halves are one tile apart).
+  uint32_t rd[kChunks];
+  {
+    const int row = lane & 15, rr = row & 7, g = lane >> 4, base = (row >> 3) * 1024 + rr * kBlock;
+    if constexpr (A16) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        rd[q] = (uint32_t)(base + (((2 * g + (q & 1)) ^ rr) << 4) + (q >> 1) * kTileBytes);
+    } else {
+      rd[0] = (uint32_t)lt.rd0;
+      rd[1] = (uint32_t)lt.rd1;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int c = 0; c < NT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < D - 1; ++s) issue_batch_weights(ring + s * St::kBytes, op, lt, w, phys(s), s < nkb);
+  issue_claim(ready);
+  wait_ready(ready);
+#pragma unroll
+  for (int s = 0; s < D - 1; ++s) issue_batch_acts(ring + s * St::kBytes, scales + s * 2048, op, w, phys(s));
+  for (int kb0 = 0; kb0 < nkb; kb0 += D) {
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+      constexpr int kAll = 8 + kAct;
+      const int kb = kb0 + s, sn = (s + D - 1) % D, kn = phys(kb + D - 1);
+      if (kb0 == 0)
+        wait_vmem<(D - 2) * kAct>();
+      else
+        wait_vmem<(D - 2) * kAll>();
+      __builtin_amdgcn_s_barrier();
+      issue_batch_weights(ring + sn * St::kBytes, op, lt, w, kn, kb + D - 1 < nkb);
+      issue_batch_acts(ring + sn * St::kBytes, scales + sn * 2048, op, w, kn);
+      if (kb < nkb) {
+        const uint32_t slot = ring_lds + s * St::kBytes;
+        const uint32_t x0 = ring_lds + kBatchRing + w * 512 + s * 2048;
+        const uint32_t pa[2] = {slot + wm * 8 * kTileBytes + lt.rd0, slot + wm * 8 * kTileBytes + lt.rd1};
+        uint32_t pb[kChunks];
+#pragma unroll
+        for (int q = 0; q < kChunks; ++q) pb[q] = slot + kBatchWeights + wn * NT * (kChunks / 2) * kTileBytes + rd[q];
+        const uint32_t px = x0 + 4 * (lane & 15);
+        i32x4 b[NT][kChunks], alo[8], ahi[8];
+        float sx[NT], k0, k1;
+        auto read_weights = [&](auto r) {
+          lds_read2<r.value * kTileBytes>(alo[r.value], ahi[r.value], pa[0], pa[1]);
+        };
+        lds_read_f<256>(k0, x0);
+        lds_read_f<260>(k1, x0);
+        static_for<0, NT>([&](auto c) {
+          if constexpr (!A16) lds_read_f<c.value * 64>(sx[c.value], px);
+          static_for<0, kChunks / 2>([&](auto h) {
+            constexpr int q = 2 * h.value;
+            lds_read2<c.value*(kChunks / 2) * kTileBytes>(b[c.value][q], b[c.value][q + 1], pb[q], pb[q + 1]);
+          });
+        });
+        static_for<0, 2 * W>(read_weights);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        static_for<0, 8 / W>([&](auto group) {
+          constexpr int r2 = W * group.value;
+          // The next W tiles' reads stay pending (none before the last).
+          lds_wait<(r2 < 8 - W ? 2 * W : 0)>(alo[r2], ahi[r2]);
+          if constexpr (W == 2) lds_arrived(alo[r2 + 1], ahi[r2 + 1]);
+          if constexpr (r2 == 0) {
+            lds_arrived(k0);
+            lds_arrived(k1);
+#pragma unroll
+            for (int c = 0; c < NT; ++c) {
+#pragma unroll
+              for (int q = 0; q < kChunks; q += 2) lds_arrived(b[c][q], b[c][q + 1]);
+              if constexpr (!A16) lds_arrived(sx[c]);
+            }
+          }
+#pragma unroll
+          for (int r = r2; r < r2 + W; ++r) {
+            const float kw = r < 4 ? k0 : k1;
+            if constexpr (A16) {
+              i32x4 a[4];
+              a[0] = e4m3x8_to_bf16(alo[r][0], alo[r][1]);
+              a[1] = e4m3x8_to_bf16(alo[r][2], alo[r][3]);
+              a[2] = e4m3x8_to_bf16(ahi[r][0], ahi[r][1]);
+              a[3] = e4m3x8_to_bf16(ahi[r][2], ahi[r][3]);
+              f32x4 p[NT];
+#pragma unroll
+              for (int c = 0; c < NT; ++c) p[c] = zero;
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int c = 0; c < NT; ++c)
+                  p[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[q]),
+                                                                 __builtin_bit_cast(bf16x8, b[c][q]), p[c], 0, 0, 0);
+#pragma unroll
+              for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[r][c][v] = __builtin_fmaf(p[c][v], kw, acc[r][c][v]);
+            } else {
+              const i32x8 ar = __builtin_shufflevector(alo[r], ahi[r], 0, 1, 2, 3, 4, 5, 6, 7);
+              f32x4 p[NT];
+#pragma unroll
+              for (int c = 0; c < NT; ++c)
+                p[c] = mfma_e4m3(ar, __builtin_shufflevector(b[c][0], b[c][1], 0, 1, 2, 3, 4, 5, 6, 7), zero);
+#pragma unroll
+              for (int c = 0; c < NT; ++c) {
+                const float k = kw * sx[c];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[r][c][v] = __builtin_fmaf(p[c][v], k, acc[r][c][v]);
+              }
+            }
+          }
+          if constexpr (r2 + 2 * W < 8) static_for<r2 + 2 * W, r2 + 3 * W>(read_weights);
+        });
+      }
+    }
+  }
+  // The tail requested stages past the end: every wave waits for its loads and the workgroup
+  // passes a barrier before any of this LDS is reused.
+  wait_vmem<0>();
+  __builtin_amdgcn_s_barrier();
+}
+
 // Row r's token: perm[row0 + r] / K (grouped rows), else row0 + r.
 __device__ __forceinline__ int row_token(const ChunkRows& cr, int r) {
   return cr.perm ? cr.perm[cr.row0 + r] / cr.K : cr.row0 + r;
@@ -2049,40 +2308,23 @@ struct GateUpArgs {
   uint16_t* h16_s;              // W8A16: of the shared rows [T, S*I]
 };
 
-// One gate/up unit: rows [jb*128, jb*128+128) of gate and of up against the chunk's
-// activation rows (at most 16*NCT). Wave w owns gate and up rows 32w .. 32w+31 of the
-// block, so SwiGLU pairs matching registers; the per-row amax over the 128-block for the
-// requantization of h is reduced across the four wavefronts through LDS.
-template <int NCT>
-__device__ __forceinline__ void gateup_unit(const GateUpArgs& a, const uint8_t* wg, const uint8_t* wu, const float* sg,
-                            const float* su, const ChunkRows& cr, int jb, uint8_t* hq, float* hs, int ldh,
-                            int rot, float (*red)[64], uint8_t* ring, const ReadyWait& ready) {
-  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kofs = 16 * (lane >> 4);
-  const int H = a.H, nkb = H / kBlock, nbh = scale_ld(ldh / kBlock);
-  Operands<4, NCT, 2> op;
-  op.lda = H;
-  op.spare = a.spare;
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const size_t row = (size_t)(32 * w + 16 * r);
-    op.a[r] = wg + row * H;
-    op.a[r + 2] = wu + row * H;
-  }
-  op.sw[0] = sg;
-  op.sw[1] = su;
-  int orow[NCT];  // the h row of each column (a padding column's is never stored)
-#pragma unroll
-  for (int c = 0; c < NCT; ++c) {
-    const int r = min(16 * c + (lane & 15), cr.n - 1);  // padding columns repeat a valid row
-    const int tok = row_token(cr, r);
-    op.b[c] = a.xq + (size_t)tok * H + kofs;
-    op.sx[c] = a.xs + (size_t)tok * nkb;
-    orow[c] = cr.by_token ? cr.out_base + tok : cr.row0 + r;
-  }
-  f32x4 acc[4][NCT];
-  stream_gemm<4, NCT, 2, 2>(op, nkb, rot, ring, acc, ready);
+// h (a bf16 value) of one element's fp32 gate and up sums: g, u = bf16 (frontier.py:184-186),
+// clamped at the SwiGLU limit L (glm53.py:175; infinity: none); h = bf16(silu(fp32 g) * fp32 u)
+// (frontier.py:337, DeepSeek) or bf16(bf16(silu(g)) * u) (frontier.py:338, glm53.py:174-175).
+__device__ __forceinline__ float swiglu_h(float gate, float up, float L, bool bf16_silu) {
+  const float g = fminf(round_bf16(gate), L);
+  const float u = fminf(fmaxf(round_bf16(up), -L), L);
+  return bf16_silu ? round_bf16(round_bf16(silu(g)) * u) : round_bf16(silu(g) * u);
+}
 
+// The gate/up epilogue of the W8A8 form: acc[0..1] gate and acc[2..3] up of the wave's two row
+// tiles, every column tile; h is requantized to E4M3 per 128 and stored to the rows orow.
+template <int NCT>
+__device__ __forceinline__ void gateup_epilogue(const GateUpArgs& a, const f32x4 (&acc)[4][NCT], const ChunkRows& cr,
+                                                const int (&orow)[NCT], int jb, uint8_t* hq, float* hs, int ldh,
+                                                float (*red)[64]) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nbh = scale_ld(ldh / kBlock);
   // g, u = bf16 (frontier.py:184-186), clamped at the SwiGLU limit if one is set
   // (glm53.py:175); h = bf16(silu(fp32 g) * fp32 u) (frontier.py:337, DeepSeek) or
   // bf16(bf16(silu(g)) * u) (frontier.py:338, glm53.py:174-175).
@@ -2125,6 +2367,70 @@ __device__ __forceinline__ void gateup_unit(const GateUpArgs& a, const uint8_t* 
   }
 }
 
+// One gate/up unit: rows [jb*128, jb*128+128) of gate and of up against the chunk's
+// activation rows (at most 16*NCT). Wave w owns gate and up rows 32w .. 32w+31 of the
+// block, so SwiGLU pairs matching registers; the per-row amax over the 128-block for the
+// requantization of h is reduced across the four wavefronts through LDS.
+template <int NCT>
+__device__ __forceinline__ void gateup_unit(const GateUpArgs& a, const uint8_t* wg, const uint8_t* wu, const float* sg,
+                            const float* su, const ChunkRows& cr, int jb, uint8_t* hq, float* hs, int ldh,
+                            int rot, float (*red)[64], uint8_t* ring, const ReadyWait& ready) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kofs = 16 * (lane >> 4);
+  const int H = a.H, nkb = H / kBlock;
+  Operands<4, NCT, 2> op;
+  op.lda = H;
+  op.spare = a.spare;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const size_t row = (size_t)(32 * w + 16 * r);
+    op.a[r] = wg + row * H;
+    op.a[r + 2] = wu + row * H;
+  }
+  op.sw[0] = sg;
+  op.sw[1] = su;
+  int orow[NCT];  // the h row of each column (a padding column's is never stored)
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    const int r = min(16 * c + (lane & 15), cr.n - 1);  // padding columns repeat a valid row
+    const int tok = row_token(cr, r);
+    op.b[c] = a.xq + (size_t)tok * H + kofs;
+    op.sx[c] = a.xs + (size_t)tok * nkb;
+    orow[c] = cr.by_token ? cr.out_base + tok : cr.row0 + r;
+  }
+  f32x4 acc[4][NCT];
+  stream_gemm<4, NCT, 2, 2>(op, nkb, rot, ring, acc, ready);
+
+  gateup_epilogue<NCT>(a, acc, cr, orow, jb, hq, hs, ldh, red);
+}
+
+// The gate/up epilogue of the W8A16 form: h stays in bf16.
+template <int NCT>
+__device__ __forceinline__ void gateup_epilogue16(const GateUpArgs& a, const f32x4 (&acc)[4][NCT],
+                                                  const ChunkRows& cr, const int (&orow)[NCT], int jb, uint16_t* h,
+                                                  int ldh) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool bf16_silu = a.swiglu != 0;
+  const float L = a.limit > 0.0f ? a.limit : INFINITY;
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    if (16 * c + (lane & 15) >= cr.n) continue;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      uint32_t bits[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float g = fminf(round_bf16(acc[p][c][v]), L);
+        const float u = fminf(fmaxf(round_bf16(acc[p + 2][c][v]), -L), L);
+        bits[v] = f32_to_bf16_bits(bf16_silu ? round_bf16(silu(g)) * u : silu(g) * u);
+      }
+      uint16_t* dst = h + (size_t)orow[c] * ldh + (size_t)jb * kBlock + 32 * w + 16 * p + 4 * (lane >> 4);
+      store_coherent(reinterpret_cast<uint64_t*>(dst),
+                     (uint64_t)(bits[0] | (bits[1] << 16)) | ((uint64_t)(bits[2] | (bits[3] << 16)) << 32));
+    }
+  }
+}
+
 // The W8A16 gate/up unit (frontier.py:180-183 with quantize=False, the expert GEMMs of the
 // DeepSeek family at frontier.py:265-270): gateup_unit's rows and waves, with the bf16 rows
 // of x as the activations; g and u are rounded to bf16 (frontier.py:183), clamped if a
@@ -2159,25 +2465,7 @@ __device__ __forceinline__ void gateup_unit16(const GateUpArgs& a, const uint8_t
   }
   f32x4 acc[4][NCT];
   stream_gemm<4, NCT, 2, 2, true>(op, H / kBlock, rot, ring, acc, ready);
-  const bool bf16_silu = a.swiglu != 0;
-  const float L = a.limit > 0.0f ? a.limit : INFINITY;
-#pragma unroll
-  for (int c = 0; c < NCT; ++c) {
-    if (16 * c + (lane & 15) >= cr.n) continue;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      uint32_t bits[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float g = fminf(round_bf16(acc[p][c][v]), L);
-        const float u = fminf(fmaxf(round_bf16(acc[p + 2][c][v]), -L), L);
-        bits[v] = f32_to_bf16_bits(bf16_silu ? round_bf16(silu(g)) * u : silu(g) * u);
-      }
-      uint16_t* dst = h + (size_t)orow[c] * ldh + (size_t)jb * kBlock + 32 * w + 16 * p + 4 * (lane >> 4);
-      store_coherent(reinterpret_cast<uint64_t*>(dst),
-                     (uint64_t)(bits[0] | (bits[1] << 16)) | ((uint64_t)(bits[2] | (bits[3] << 16)) << 32));
-    }
-  }
+  gateup_epilogue16<NCT>(a, acc, cr, orow, jb, h, ldh);
 }
 
 // Gate/up unit u of the work list (of the dense schedule's lists): chunk u / nbI, 128-row
@@ -2193,7 +2481,7 @@ __device__ __forceinline__ void gateup_work(const GateUpArgs& a, int u, float (*
   const int nbI = a.I / kBlock, nkb = a.H / kBlock;
   const int4 ch = a.dense ? dense_gu_chunk(u / nbI, a.E, a.S, a.T, nbI) : a.chunks[u / nbI];
   const int j = u % nbI, jb = ch.w + j;
-  const int rot = u % nkb;  // concurrent units start at different K blocks
+  const int rot = (ch.x * nbI + jb) % nkb;  // keyed by the weight block (see stream_gemm)
   const uint8_t *wg, *wu;
   const float *sg, *su;
   uint8_t* hq;
@@ -2235,6 +2523,137 @@ __device__ __forceinline__ void gateup_work(const GateUpArgs& a, int u, float (*
   } else {
     gateup_unit<4>(a, wg, wu, sg, su, cr, jb, hq, hs, ldh, rot, red, ring, ready);
   }
+}
+
+// The batch gate/up unit: 128 rows of gate and of up (jb) against a chunk of at most 32*NT rows.
+// Weight tiles 0-3 of wave pair wm are gate rows 64wm .. +63, tiles 4-7 the same rows of up, so
+// SwiGLU pairs matching registers; the amax of a row's 128-block is taken over the two waves that
+// hold its columns. Each output's sum runs over the K blocks in gateup_unit's order.
+template <int NT, bool A16>
+__device__ __forceinline__ void gateup_batch_unit(const GateUpArgs& a, const uint8_t* wg, const uint8_t* wu,
+                                                  const float* sg, const float* su, const ChunkRows& cr, int jb,
+                                                  uint8_t* hq, float* hs, uint16_t* h16, int ldh, int rot,
+                                                  float* red, uint8_t* ring, const ReadyWait& ready) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = w & 1, c0 = (w >> 1) * 16 * NT;  // this wave's row half and first column
+  const int H = a.H, nkb = H / kBlock, nbh = scale_ld(ldh / kBlock);
+  BatchOperands<NT, A16> op;
+  op.lda = H;
+  op.spare = a.spare;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) op.a[i] = (w & 1 ? wu : wg) + (size_t)(64 * (w >> 1) + 16 * i) * H;
+  op.sw = lane & 1 ? su : sg;
+  const auto token = [&cr](int r) { return row_token(cr, r); };
+  batch_rows(op, A16 ? reinterpret_cast<const uint8_t*>(a.x16) : a.xq, (size_t)H * (A16 ? 2 : 1), cr.n, token);
+  op.sx = A16 ? nullptr : a.xs + (size_t)token(min(c0 + (lane & (16 * NT - 1)), cr.n - 1)) * nkb;
+  f32x4 acc[8][NT];
+  stream_gemm_batch<NT, A16>(op, nkb, rot, ring, acc, ready);
+  const bool bf16_silu = a.swiglu != 0;
+  const float L = a.limit > 0.0f ? a.limit : INFINITY;
+  const int hcol = jb * kBlock + 64 * wm + 4 * (lane >> 4);  // + 16p: this lane's h columns
+  if constexpr (!A16) {
+    // red[wm][row]: the amax of each row over the pair's 64 channels.
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+      float amax = 0.0f;
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float h = swiglu_h(acc[p][c][v], acc[p + 4][c][v], L, bf16_silu);
+          acc[p][c][v] = h;
+          amax = fmaxf(amax, fabsf(h));
+        }
+      amax = fmaxf(amax, __shfl_xor(amax, 16));
+      amax = fmaxf(amax, __shfl_xor(amax, 32));
+      if (lane < 16) red[wm * 128 + c0 + 16 * c + lane] = amax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+      const int r = c0 + 16 * c + (lane & 15);
+      const float s = act_scale(fmaxf(red[r], red[128 + r]), a.pow2);
+      if (r < cr.n) {
+        uint8_t* dst = hq + (size_t)(cr.row0 + r) * ldh + hcol;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          store_coherent(reinterpret_cast<uint32_t*>(dst + 16 * p),
+                         e4m3x4(clamp448(acc[p][c][0] / s), clamp448(acc[p][c][1] / s), clamp448(acc[p][c][2] / s),
+                                clamp448(acc[p][c][3] / s)));
+        if (wm == 0 && lane < 16) store_coherent(hs + (size_t)(cr.row0 + r) * nbh + jb, s);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+      const int r = c0 + 16 * c + (lane & 15);
+      if (r < cr.n) {
+        uint16_t* dst = h16 + (size_t)(cr.row0 + r) * ldh + hcol;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          uint32_t bits[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            bits[v] = __float_as_uint(swiglu_h(acc[p][c][v], acc[p + 4][c][v], L, bf16_silu)) >> 16;
+          store_coherent(reinterpret_cast<uint64_t*>(dst + 16 * p),
+                         (uint64_t)(bits[0] | (bits[1] << 16)) | ((uint64_t)(bits[2] | (bits[3] << 16)) << 32));
+        }
+      }
+    }
+  }
+}
+
+// Gate/up unit u of the batch form: gateup_work's over chunks of at most 128 rows (no dense schedule).
+template <bool A16>
+__device__ __forceinline__ void gateup_batch_work(const GateUpArgs& a, int u, float* red, uint8_t* ring,
+                                                  const ReadyWait& ready) {
+  const int nbI = a.I / kBlock, nkb = a.H / kBlock;
+  const int4 ch = a.chunks[u / nbI];
+  const bool shared = ch.x == a.E;
+  const int jb = ch.w + u % nbI;
+  const int rot = (ch.x * nbI + jb) % nkb;
+  const uint8_t *wg, *wu;
+  const float *sg, *su;
+  uint8_t* hq;
+  float* hs;
+  uint16_t* h16;
+  const int* perm;
+  int ldh;
+  size_t rowblk;
+  if (shared) {
+    rowblk = (size_t)jb;
+    wg = a.sgate;
+    wu = a.sup;
+    sg = a.sgate_scale;
+    su = a.sup_scale;
+    hq = a.hq_s;
+    hs = a.hs_s;
+    h16 = a.h16_s;
+    perm = nullptr;
+    ldh = a.S * a.I;
+  } else {
+    rowblk = (size_t)ch.x * nbI + jb;
+    wg = a.gate;
+    wu = a.up;
+    sg = a.gate_scale;
+    su = a.up_scale;
+    hq = a.hq_r;
+    hs = a.hs_r;
+    h16 = a.h16_r;
+    perm = a.perm;
+    ldh = a.I;
+  }
+  wg += rowblk * kBlock * a.H;
+  wu += rowblk * kBlock * a.H;
+  sg += rowblk * nkb;
+  su += rowblk * nkb;
+  const ChunkRows cr{ch.z, ch.y, perm, a.K};
+  if (cr.n <= 32)
+    gateup_batch_unit<1, A16>(a, wg, wu, sg, su, cr, jb, hq, hs, h16, ldh, rot, red, ring, ready);
+  else if (cr.n <= 64)
+    gateup_batch_unit<2, A16>(a, wg, wu, sg, su, cr, jb, hq, hs, h16, ldh, rot, red, ring, ready);
+  else
+    gateup_batch_unit<4, A16>(a, wg, wu, sg, su, cr, jb, hq, hs, h16, ldh, rot, red, ring, ready);
 }
 
 // One half of a gate/up block: rows [jb*128, jb*128+128) of gate (half 0) or of up (half 1)
@@ -2423,6 +2842,41 @@ struct DownArgs {
   const uint16_t* h16_s;  // W8A16: of the shared rows [T, S*I]
 };
 
+// Stores a wave's RT row tiles (from output channel h0) of a down unit: d in bf16, or with
+// several K parts the fp32 partial.
+template <int RT, int NCT, bool CO>
+__device__ __forceinline__ void down_epilogue(const DownArgs& a, const f32x4 (&acc)[RT][NCT], const ChunkRows& cr,
+                                              const int (&orow)[NCT], int h0, uint16_t* d, float* pd) {
+  const int lane = opaque_lane();
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    const int r = 16 * c + (lane & 15);
+    if (r < cr.n) {
+#pragma unroll
+      for (int p = 0; p < RT; ++p) {
+        const size_t o = (size_t)orow[c] * a.H + h0 + 16 * p + 4 * (lane >> 4);
+        // Device-coherent stores: the combine (a later kernel, or a later unit of the
+        // single-launch kernel on another XCD) reads them.
+        if (a.ks == 1) {
+          const uint32_t lo = f32_to_bf16_bits(acc[p][c][0]) | (f32_to_bf16_bits(acc[p][c][1]) << 16);
+          const uint32_t hi = f32_to_bf16_bits(acc[p][c][2]) | (f32_to_bf16_bits(acc[p][c][3]) << 16);
+          store_out<CO>(reinterpret_cast<uint64_t*>(d + o), (uint64_t)lo | ((uint64_t)hi << 32));
+        } else {
+          uint64_t* q = reinterpret_cast<uint64_t*>(pd + o);
+          store_out<CO>(q, (uint64_t)__float_as_uint(acc[p][c][0]) | ((uint64_t)__float_as_uint(acc[p][c][1]) << 32));
+          store_out<CO>(q + 1, (uint64_t)__float_as_uint(acc[p][c][2]) | ((uint64_t)__float_as_uint(acc[p][c][3]) << 32));
+        }
+      }
+    }
+  }
+}
+
+// The K rotation of the down units of one 256-row block (two 128-row units, or one batch unit)
+// and K part: keyed by the weights, so a row's sums do not depend on the form that computes them.
+__device__ __forceinline__ int down_rotation(int e, int j2, int kp, int H, int I, int ks) {
+  return ((e * ((H / kBlock + 1) / 2) + j2) * ks + kp) % (I / kBlock / ks);
+}
+
 // One down unit: rows [j*128, j*128+128) of a down matrix [H, ldk] against the chunk's
 // requantized h rows, over K part kp of a.ks (K blocks [kp*nkb/ks, (kp+1)*nkb/ks)). Wave w
 // owns rows 32w .. 32w+31. With one part the result is d in bf16; with several, each part
@@ -2471,27 +2925,7 @@ __device__ __forceinline__ void down_unit(const DownArgs& a, const uint8_t* wd, 
   } else {
     stream_gemm<2, NCT, 1, 4>(op, nkbp, rot, ring, acc, ready);
   }
-#pragma unroll
-  for (int c = 0; c < NCT; ++c) {
-    const int r = 16 * c + (lane & 15);
-    if (r < cr.n) {
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const size_t o = (size_t)orow[c] * a.H + (size_t)j * kBlock + 32 * w + 16 * p + 4 * (lane >> 4);
-        // Device-coherent stores: the combine (a later kernel, or a later unit of the
-        // single-launch kernel on another XCD) reads them.
-        if (a.ks == 1) {
-          const uint32_t lo = f32_to_bf16_bits(acc[p][c][0]) | (f32_to_bf16_bits(acc[p][c][1]) << 16);
-          const uint32_t hi = f32_to_bf16_bits(acc[p][c][2]) | (f32_to_bf16_bits(acc[p][c][3]) << 16);
-          store_out<CO>(reinterpret_cast<uint64_t*>(d + o), (uint64_t)lo | ((uint64_t)hi << 32));
-        } else {
-          uint64_t* q = reinterpret_cast<uint64_t*>(pd + o);
-          store_out<CO>(q, (uint64_t)__float_as_uint(acc[p][c][0]) | ((uint64_t)__float_as_uint(acc[p][c][1]) << 32));
-          store_out<CO>(q + 1, (uint64_t)__float_as_uint(acc[p][c][2]) | ((uint64_t)__float_as_uint(acc[p][c][3]) << 32));
-        }
-      }
-    }
-  }
+  down_epilogue<2, NCT, CO>(a, acc, cr, orow, j * kBlock + 32 * w, d, pd);
 }
 
 // Down unit v of the work list: chunk v / (nbH*ks), then 128-row block j of the down
@@ -2505,7 +2939,7 @@ __device__ __forceinline__ void down_work(const DownArgs& a, int v, const ReadyW
   const int c = v / (nbH * a.ks);
   const int4 ch = a.dense ? dense_dn_chunk(c, a.E, a.S, a.T) : a.chunks[c];
   const int rem = v % (nbH * a.ks), j = rem / a.ks, kp = rem % a.ks;
-  const int rot = v % (nbI / a.ks);  // concurrent units start at different K blocks
+  const int rot = down_rotation(ch.x, j >> 1, kp, a.H, a.I, a.ks);
   float* pd_s = a.p_s + (size_t)kp * a.T * a.H;
   float* pd_r = a.p_r + (size_t)kp * a.rows_r * a.H;
   if (ch.x == a.E) {
@@ -2549,6 +2983,80 @@ __device__ __forceinline__ void down_work(const DownArgs& a, int v, const ReadyW
     else
       down_unit<4, CO>(a, wd, sd, a.I, a.hq_r, a.hs_r, cr, j, kp, a.d_r, pd_r, rot, ready, ring);
   }
+}
+
+// The batch down unit: 256 rows of a down matrix (two 128-row blocks, one per wave pair wm) against
+// a chunk of at most 32*NT rows. A row's sums are down_unit's (the same K blocks in the same order).
+template <int NT, bool A16>
+__device__ __forceinline__ void down_batch_unit(const DownArgs& a, const uint8_t* wd, const float* sd, int ldk,
+                                                const uint8_t* hq, const float* hs, const ChunkRows& cr, int j2,
+                                                int kp, uint16_t* d, float* pd, int rot, const ReadyWait& ready,
+                                                uint8_t* ring) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = w & 1, c0 = (w >> 1) * 16 * NT;
+  const int nkb = ldk / kBlock, nkbp = nkb / a.ks, kb0 = kp * nkbp, ld = ldk * (A16 ? 2 : 1);
+  BatchOperands<NT, A16> op;
+  op.lda = ldk;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) op.a[i] = wd + (size_t)(64 * w + 16 * i) * ldk + (size_t)kb0 * kBlock;
+  op.spare = a.spare;
+  op.sw = sd + (size_t)wm * nkb + kb0;
+  batch_rows(op, hq + (size_t)cr.row0 * ld + (size_t)kb0 * kBlock * (A16 ? 2 : 1), (size_t)ld, cr.n,
+             [](int r) { return r; });
+  op.sx = A16 ? nullptr
+              : hs + (size_t)(cr.row0 + min(c0 + (lane & (16 * NT - 1)), cr.n - 1)) * scale_ld(nkb) + kb0;
+  f32x4 acc[8][NT];
+  stream_gemm_batch<NT, A16>(op, nkbp, rot, ring, acc, ready);
+  // down_epilogue counts rows of a chunk from its first column on.
+  const ChunkRows mine{cr.n - c0, cr.row0 + c0, nullptr, cr.K};
+  int orow[NT];
+#pragma unroll
+  for (int c = 0; c < NT; ++c) orow[c] = mine.row0 + 16 * c + (lane & 15);
+  down_epilogue<8, NT, true>(a, acc, mine, orow, j2 * 2 * kBlock + 128 * wm, d, pd);
+}
+
+// Down unit v of the batch form: chunk v / (nbH/2*ks), then 256-row block j2 and K part kp.
+template <bool A16>
+__device__ __forceinline__ void down_batch_work(const DownArgs& a, int v, const ReadyWait& ready, uint8_t* ring) {
+  const int nbH2 = a.H / (2 * kBlock), nbI = a.I / kBlock;
+  const int4 ch = a.chunks[v / (nbH2 * a.ks)];
+  const int rem = v % (nbH2 * a.ks), j2 = rem / a.ks, kp = rem % a.ks;
+  const bool shared = ch.x == a.E;
+  const int rot = down_rotation(ch.x, j2, kp, a.H, a.I, a.ks);
+  const uint8_t *wd, *hq;
+  const float *sd, *hs;
+  uint16_t* d;
+  float* pd;
+  int ldk;
+  size_t blk;
+  if (shared) {
+    ldk = a.S * a.I;
+    blk = (size_t)2 * j2;
+    wd = a.sdown;
+    sd = a.sdown_scale;
+    hq = A16 ? reinterpret_cast<const uint8_t*>(a.h16_s) : a.hq_s;
+    hs = a.hs_s;
+    d = a.d_s;
+    pd = a.p_s + (size_t)kp * a.T * a.H;
+  } else {
+    ldk = a.I;
+    blk = (size_t)ch.x * (a.H / kBlock) + 2 * j2;
+    wd = a.down;
+    sd = a.down_scale;
+    hq = A16 ? reinterpret_cast<const uint8_t*>(a.h16_r) : a.hq_r;
+    hs = a.hs_r;
+    d = a.d_r;
+    pd = a.p_r + (size_t)kp * a.rows_r * a.H;
+  }
+  wd += blk * kBlock * ldk;
+  sd += blk * (ldk / kBlock);
+  const ChunkRows cr{ch.z, ch.y, nullptr, a.K};
+  if (cr.n <= 32)
+    down_batch_unit<1, A16>(a, wd, sd, ldk, hq, hs, cr, j2, kp, d, pd, rot, ready, ring);
+  else if (cr.n <= 64)
+    down_batch_unit<2, A16>(a, wd, sd, ldk, hq, hs, cr, j2, kp, d, pd, rot, ready, ring);
+  else
+    down_batch_unit<4, A16>(a, wd, sd, ldk, hq, hs, cr, j2, kp, d, pd, rot, ready, ring);
 }
 
 // y[t, h0 .. h0+7] = bf16( sum_slot fp32(d[t,slot]) * w[t,slot]  (slot order, each product
@@ -3083,17 +3591,28 @@ __device__ __forceinline__ int dense_state(int* ctl, const int* offsets, int e, 
   return st;
 }
 
+// LDS of k_layer beside the rings.
+struct LayerMisc {
+  float red[4][64];
+  double part[4];
+  int slot, flag, flags[2], units[2];
+};
+
 // A16: the W8A16 form (bf16 activations into the expert units, chunks of at most 32 rows).
-template <bool SPLIT, bool A16 = false>
-__global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
+// BATCH: the batch units (gateup_batch_work, down_batch_work).
+template <bool SPLIT, bool A16, bool BATCH>
+__device__ __forceinline__ void layer_body(const LayerArgs& args) {
   typedef const __attribute__((address_space(4))) LayerArgs* ArgsPtr;
   typedef const __attribute__((address_space(4))) ExpertArgs* ExArgsPtr;
-  __shared__ float red[4][64];
-  __shared__ __attribute__((aligned(16))) uint8_t rings[4 * kRingWave];  // weight rings; front-end scratch
-  __shared__ int slot, flag, flags[2], units[2];
-  __shared__ double part[4];
+  // Weight rings, in the batch form the slots of whole stages; front-end scratch.
+  __shared__ __attribute__((aligned(16))) uint8_t rings[BATCH ? kBatchRing + kBatchScales : 4 * kRingWave];
+  __shared__ LayerMisc misc;
+  float(*red)[64] = misc.red;
+  int &slot = misc.slot, &flag = misc.flag;
+  int *flags = misc.flags, *units = misc.units;
+  double* part = misc.part;
   static_assert(sizeof(LayerArgs) % 8 == 0 && offsetof(LayerArgs, ex) == 0, "argument segment layout");
-  static_assert(sizeof(SelectLds) <= sizeof(rings) && (kRouterWaves - 1) * 4 * 64 * sizeof(f64x4) <= sizeof(rings),
+  static_assert(sizeof(SelectLds) <= 4 * kRingWave && (kRouterWaves - 1) * 4 * 64 * sizeof(f64x4) <= 4 * kRingWave,
                 "front-end scratch in the rings");
   int* ctl = args.ctl;
   const int fixed = args.n_norm + args.n_router + args.T;  // units listed before the routing is known
@@ -3197,8 +3716,8 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
       if (publish_count(ctl, kCtlSelected, 1, a.T, -1, &units[0]) == a.T - 1) {
         // Every token is routed: this workgroup runs the permute, then publishes the lists.
         acquire_after_wait();
-        permute_block<true>(a.ids, 0, a.T, a.K, a.E, a.S, a.ex.gu.I / kBlock, a.H / kBlock, a.ks,
-                            A16 ? kChunkRowsA16 : kChunkRows, 0,
+        permute_block<true>(a.ids, 0, a.T, a.K, a.E, a.S, a.ex.gu.I / kBlock, a.H / kBlock / (BATCH ? 2 : 1), a.ks,
+                            BATCH ? kChunkRowsBatch : (A16 ? kChunkRowsA16 : kChunkRows), 0,
                             a.po, reinterpret_cast<int*>(rings), flags,
                             permute_tile_waves(a.T, a.E, 256, kPermuteLdsInts));
         publish_fence();
@@ -3225,7 +3744,7 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
   // Kimi-K2 0, over two A/B runs; 16 naps measured no better).
   // The dense schedule's lists are known from the geometry: no wait (its units wait for the
   // quantized x and for each other instead; the combine for the routing).
-  const bool dense = args.dense != 0;
+  const bool dense = !BATCH && args.dense != 0;
   if (!dense) {
     if (args.ex.gu.S > 0) touch_shared_weights(args.ex, blockIdx.x, gridDim.x);
     wait_ready(ReadyWait{my_signal_flag(ctl, kSigPermuted), 1, &ctl[kCtlError], kWaitTicks, true, 8});
@@ -3264,6 +3783,8 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
       bool done = true;
       if constexpr (SPLIT) {
         done = gateup_work_split(a.gu, g, red, &flag, ring, claiming(ReadyWait{nullptr, 0, nullptr}, queue, &ticket));
+      } else if constexpr (BATCH) {
+        gateup_batch_work<A16>(a.gu, g, &red[0][0], rings, claiming(ReadyWait{nullptr, 0, nullptr}, queue, &ticket));
       } else if (dense) {
         // Every expert's units from the start: before the routing is known a unit works every
         // token and waits only for the quantized x; after, its expert's routed rows, or
@@ -3285,15 +3806,17 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
         if (threadIdx.x == 0) atomicAdd(&a.ready[(size_t)dc * a.ready_stride], 1);
       }
     } else {
-      const int v = u - fixed - n_gu, c = v / (nbH * a.dn.ks);
+      const int v = u - fixed - n_gu, c = v / ((BATCH ? nbH / 2 : nbH) * a.dn.ks);
       const int sh = a.dn.S > 0 ? 1 : 0;
       const int st = dense && c >= sh ? dense_state(ctl, a.gu.offsets, c - sh, &flags[0]) : 0;
       if (st != 2) {
         const int need = dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI);
-        down_work<true, A16>(a.dn, v,
-                             claiming(ReadyWait{&a.ready[(size_t)c * a.ready_stride], need, &ctl[kCtlError]}, queue,
-                                      &ticket),
-                             ring, st == 1);
+        const ReadyWait ready = claiming(
+            ReadyWait{&a.ready[(size_t)c * a.ready_stride], need, &ctl[kCtlError]}, queue, &ticket);
+        if constexpr (BATCH)
+          down_batch_work<A16>(a.dn, v, ready, rings);
+        else
+          down_work<true, A16>(a.dn, v, ready, ring, st == 1);
       }
       ++my_down;
     }
@@ -3365,6 +3888,17 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
   }
 }
 
+template <bool SPLIT, bool A16 = false>
+__global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
+  layer_body<SPLIT, A16, false>(args);
+}
+
+// One workgroup per CU (the batch ring).
+template <bool A16>
+__global__ __launch_bounds__(256, 1) void k_layer_batch(LayerArgs args) {
+  layer_body<false, A16, true>(args);
+}
+
 // =======================================================================================
 // The MXFP4 form (megamoe.py:116-182, serial): E2M1 expert weights with one E8M0 scale per
 // 32 input channels, activations in E4M3 with E8M0 scales per 32, routing as an input.
@@ -3382,16 +3916,6 @@ __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
 // =======================================================================================
 
 constexpr int kMxStageK = 256;
-
-// Calls f(std::integral_constant<int, I>{}) for I = B .. E-1 (a loop whose index is a
-// compile-time constant in the body).
-template <int B, int E, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
-  }
-}
 
 __device__ __forceinline__ f32x4 mfma_e2m1_e4m3(const i32x4& a, const i32x8& b, f32x4 c, int sa, int sb) {
   const i32x8 a8 = {a[0], a[1], a[2], a[3], 0, 0, 0, 0};
@@ -4639,6 +5163,21 @@ bool split_gate_up(const megamoe_desc& d) {
   return units < 512 && d.hidden / kBlock >= 32;
 }
 
+// Whether the single launch works batch units (k_layer_batch: 256 weight rows by up to 128
+// activation rows through LDS, one workgroup per CU) or the decode units (16-64 rows, two). The
+// decode units stream weights faster while an expert's rows are few (their waves share nothing);
+// past about 16 rows an expert they are bound by activation loads, and past 64 (W8A16: 32) they
+// stream an expert's weights more than once. One call, decode units -> batch units: DeepSeek-V3's
+// shape at 64 / 256 / 512 tokens 767 -> 788, 1165 -> 1105, 1569 -> 1342 us (W8A16 788 -> 824,
+// 1397 -> 1193, 2209 -> 1555), Mixtral's at 64 / 256 / 512 310 -> 278, 559 -> 386, 908 -> 586,
+// Qwen3-30B-A3B's at 128 / 256 / 512 149 -> 158, 181 -> 176, 231 -> 218. Depends on the geometry
+// only; both give the same bits (the separate gate and up units, whose K rotations differ, keep
+// their geometries).
+bool batch_units(const megamoe_desc& d) {
+  return !dense_experts(d) && d.hidden % (2 * kBlock) == 0 &&
+         (d.tokens >= 256 || (int64_t)d.tokens * d.topk >= (int64_t)16 * d.experts);
+}
+
 Layout make_layout(const megamoe_desc& d) {
   Layout L{};
   const size_t T = d.tokens, H = d.hidden, E = d.experts, K = d.topk, I = d.intermediate, S = d.shared_experts;
@@ -5063,13 +5602,14 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   // As many workgroups as fit on the device at once, and no more than the most units the
   // queue can hold.
   const bool split = !a16 && split_gate_up(d);
+  const bool batch = !split && batch_units(d);
   const size_t units_max = (size_t)la.n_norm + la.n_router + T +
                            expert_units_max(d, L, split, a16 ? kChunkRowsA16 : kChunkRows) +
                            ((size_t)T * H + kCombineUnit - 1) / kCombineUnit;
   la.dense = L.dense;
   la.n_ready = L.n_ready_l;
   if (L.dense) la.ex.ready = (int*)(ws + L.ready_l);
-  const size_t resident = (size_t)di.cus * di.layer_per_cu;
+  const size_t resident = (size_t)di.cus * (batch ? 1 : di.layer_per_cu);
   const unsigned grid = (unsigned)(units_max < resident ? units_max : resident);
   // Router units taken by workgroup index: the first round of them, when there are 64 or more
   // (fewer are claimed from the queue in ~1 us: Mixtral's 8 measured 2 us slower by index);
@@ -5079,7 +5619,11 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   const char* rescue = getenv("MEGAMOE_FORCE_RESCUE");
   la.force_rescue = rescue && rescue[0] == '1' ? 1 : 0;
   if (mark(0) != hipSuccess) return MEGAMOE_ERR_HIP;
-  if (a16)
+  if (a16 && batch)
+    hipLaunchKernelGGL(k_layer_batch<true>, dim3(grid), dim3(256), 0, st, la);
+  else if (batch)
+    hipLaunchKernelGGL(k_layer_batch<false>, dim3(grid), dim3(256), 0, st, la);
+  else if (a16)
     hipLaunchKernelGGL((k_layer<false, true>), dim3(grid), dim3(256), 0, st, la);
   else if (split)
     hipLaunchKernelGGL(k_layer<true>, dim3(grid), dim3(256), 0, st, la);
