@@ -36,6 +36,7 @@ def _cases():
         out.append(_case(MIXTRAL, act, tokens=300, experts=16, topk=3, hidden=768, intermediate=384))
         out.append(_case(MIXTRAL, act, tokens=70, experts=8, hidden=4096, intermediate=512))
         out.append(_case(DEEPSEEK, act, tokens=261))
+        out.append(_case(KIMI, act, tokens=213, experts=16, topk=12))  # more slots than a load round of eight
         out.append(replace(_case(DEEPSEEK, act, tokens=300, shared_experts=2), norm="fp32_weight", residual=True))
         out.append(_case(KIMI, act, tokens=500, experts=32, topk=2))  # skewed: most experts hold few rows, some none
     out.append(replace(_case(DEEPSEEK, tokens=270), swiglu="bf16", swiglu_limit=0.5, power_of_two=True))

@@ -386,6 +386,18 @@ inline int router_splits(int H) {
   return best;
 }
 
+// At batch sizes (batch_units) there are token passes enough to fill the chip: the splits halve
+// while the units exceed kRouterBatchUnits, so each unit's MFMA chain runs over more channels
+// (its start, sums and stores counted less often) and the routing adds fewer partials (16 splits of
+// 512 x 256 logits are 17 MB in fp64).
+constexpr int kRouterBatchUnits = 512;
+inline int router_splits_batch(int H, int E, int T) {
+  int n = router_splits(H);
+  const int tiles = (T + kRouterTile - 1) / kRouterTile, passes = (tiles + 3) / 4;
+  while (n > 1 && (int64_t)n * ((E + kRouterTile - 1) / kRouterTile) * passes > kRouterBatchUnits) n /= 2;
+  return n;
+}
+
 inline int router_quant_groups(int T, int H) {
   return (T * (H / kBlock) + 4 * kQuantPerWave - 1) / (4 * kQuantPerWave);
 }
@@ -417,7 +429,7 @@ __device__ __forceinline__ void quant_x_group(int group, const uint16_t* __restr
 // wavefront order through LDS and the split's partial is stored in fp64. Passes are
 // workgroups of their own, so every workgroup does the same work and the grid spreads
 // evenly over the CUs.
-template <int NTT, bool CO>
+template <int NTT, bool CO, bool PIPE>
 __device__ __forceinline__ void router_tile(const uint16_t* __restrict__ x, const float* __restrict__ w,
                                             double* __restrict__ partial, int T, int H, int E, int n_et, int nsplit,
                                             int unit, f64x4* red) {
@@ -445,34 +457,54 @@ __device__ __forceinline__ void router_tile(const uint16_t* __restrict__ x, cons
     f64x4 acc[NTT];
 #pragma unroll
     for (int i = 0; i < NTT; ++i) acc[i] = f64x4{0.0, 0.0, 0.0, 0.0};
-    for (int c0 = 0; c0 < steps; c0 += kRouterDepth) {
-    float4 a[kRouterDepth];
-    uint2 b[kRouterDepth][NTT];
-#pragma unroll
-    for (int u = 0; u < kRouterDepth; ++u) {
-      const int k = min(c0 + u, steps - 1) * 16;
-      a[u] = *reinterpret_cast<const float4*>(wp + k);
-#pragma unroll
-      for (int i = 0; i < NTT; ++i) b[u][i] = *reinterpret_cast<const uint2*>(xp[i] + k);
-    }
-#pragma unroll
-    for (int u = 0; u < kRouterDepth; ++u) {
-      const bool live = c0 + u < steps;  // steps past the end contribute zero
-      const bool ok_a = e_ok && live;
-      const float av[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const double ac = ok_a ? (double)av[c] : 0.0;
-#pragma unroll
-        for (int i = 0; i < NTT; ++i) {
-          const uint32_t word = c < 2 ? b[u][i].x : b[u][i].y;
-          const float xv = bf16_bits_to_f32((c & 1) ? (word >> 16) : (word & 0xffffu));
-          const double bc = (t_ok[i] && live) ? (double)xv : 0.0;
-          acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac, bc, acc[i], 0, 0, 0);
+    // DEPTH steps of loads, and their products; steps past the end repeat the last one's loads and
+    // contribute zero. PIPE (slices of several rounds, at the batch sizes): half the steps at a
+    // time, each half requested again for the next round while the other is multiplied.
+    constexpr int kSteps = PIPE ? kRouterDepth / 2 : kRouterDepth;
+    float4 a[PIPE ? 2 : 1][kSteps];
+    uint2 b[PIPE ? 2 : 1][kSteps][NTT];
+#define MEGAMOE_ROUTER_LOAD(half, c0)                                                            \
+  _Pragma("unroll") for (int u = 0; u < kSteps; ++u) {                                           \
+    const int k = min((c0) + u, steps - 1) * 16;                                                 \
+    a[half][u] = *reinterpret_cast<const float4*>(wp + k);                                       \
+    _Pragma("unroll") for (int i = 0; i < NTT; ++i) b[half][u][i] = *reinterpret_cast<const uint2*>(xp[i] + k); \
+  }
+#define MEGAMOE_ROUTER_MULTIPLY(half, c0)                                                        \
+  _Pragma("unroll") for (int u = 0; u < kSteps; ++u) {                                           \
+    const bool live = (c0) + u < steps;                                                          \
+    const bool ok_a = e_ok && live;                                                              \
+    const float av[4] = {a[half][u].x, a[half][u].y, a[half][u].z, a[half][u].w};                \
+    _Pragma("unroll") for (int c = 0; c < 4; ++c) {                                              \
+      const double ac = ok_a ? (double)av[c] : 0.0;                                              \
+      _Pragma("unroll") for (int i = 0; i < NTT; ++i) {                                          \
+        const uint32_t word = c < 2 ? b[half][u][i].x : b[half][u][i].y;                         \
+        const float xv = bf16_bits_to_f32((c & 1) ? (word >> 16) : (word & 0xffffu));            \
+        const double bc = (t_ok[i] && live) ? (double)xv : 0.0;                                  \
+        acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac, bc, acc[i], 0, 0, 0);                  \
+      }                                                                                          \
+    }                                                                                            \
+  }
+    if constexpr (PIPE) {
+      MEGAMOE_ROUTER_LOAD(0, 0)
+      MEGAMOE_ROUTER_LOAD(1, kSteps)
+      for (int c0 = 0;; c0 += kRouterDepth) {
+        MEGAMOE_ROUTER_MULTIPLY(0, c0)
+        if (c0 + kRouterDepth >= steps) {
+          MEGAMOE_ROUTER_MULTIPLY(1, c0 + kSteps)
+          break;
         }
+        MEGAMOE_ROUTER_LOAD(0, c0 + kRouterDepth)
+        MEGAMOE_ROUTER_MULTIPLY(1, c0 + kSteps)
+        MEGAMOE_ROUTER_LOAD(1, c0 + kRouterDepth + kSteps)
+      }
+    } else {
+      for (int c0 = 0; c0 < steps; c0 += kRouterDepth) {
+        MEGAMOE_ROUTER_LOAD(0, c0)
+        MEGAMOE_ROUTER_MULTIPLY(0, c0)
       }
     }
-    }
+#undef MEGAMOE_ROUTER_LOAD
+#undef MEGAMOE_ROUTER_MULTIPLY
     // Slices of the split, added in wavefront order.
     if (wv > 0) {
 #pragma unroll
@@ -509,7 +541,7 @@ __global__ __launch_bounds__(kRouterWaves * 64) void k_router(const uint16_t* __
                                                               double* __restrict__ partial, int T, int H, int E,
                                                               int n_et, int nsplit) {
   __shared__ f64x4 red[(kRouterWaves - 1) * NTT * 64];
-  router_tile<NTT, false>(x, w, partial, T, H, E, n_et, nsplit, blockIdx.x, red);
+  router_tile<NTT, false, true>(x, w, partial, T, H, E, n_et, nsplit, blockIdx.x, red);
 }
 
 // logits[t][e] = fp32(sum of the splits in split order); used by megamoe_router_logits.
@@ -664,6 +696,35 @@ __device__ __forceinline__ void quant_row(const uint16_t* x, uint8_t* xq, float*
   __syncthreads();
 }
 
+// quant_row by one wavefront (the batch form's routing units: a row per wavefront).
+__device__ __forceinline__ void quant_row_wave(const uint16_t* x, uint8_t* xq, float* xs, int nbh, int pow2,
+                                               int lane) {
+  constexpr int kPairs = 4;
+  const int l = lane & 31, half = lane >> 5;
+  for (int b0 = 0; b0 < nbh; b0 += 2 * kPairs) {
+    uint2 four[kPairs];
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j)
+      four[j] = *reinterpret_cast<const uint2*>(x + (size_t)min(b0 + 2 * j + half, nbh - 1) * kBlock + 4 * l);
+    uint32_t m[kPairs];
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j) m[j] = half_wave_max_u32(bf16x4_absmax_bits(four[j]));
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j) {
+      const int b = b0 + 2 * j + half;
+      const float s = act_scale(__uint_as_float(m[j] << 16), pow2);
+      const uint32_t q = e4m3x4(clamp448(bf16_bits_to_f32(four[j].x & 0xffffu) / s),
+                                clamp448(bf16_bits_to_f32(four[j].x >> 16) / s),
+                                clamp448(bf16_bits_to_f32(four[j].y & 0xffffu) / s),
+                                clamp448(bf16_bits_to_f32(four[j].y >> 16) / s));
+      if (b < nbh) {
+        store_coherent(reinterpret_cast<uint32_t*>(xq + (size_t)b * kBlock + 4 * l), q);
+        if (l == 0) store_coherent(xs + b, s);
+      }
+    }
+  }
+}
+
 // Merges the (largest, second largest) pairs of lanes at butterfly step STEP.
 template <int STEP>
 __device__ __forceinline__ void top2_step(float& b1, float& b2) {
@@ -695,18 +756,20 @@ __device__ __forceinline__ unsigned long long select_key(float score, int e) {
 // Tokens per workgroup: one. Its four wavefronts load and sum the split partials of the
 // token's logits (one entry, all splits, per thread for up to 256 experts), then
 // wavefront 0 routes the token.
-constexpr int kSelectTokens = 1;
+constexpr int kSelectTokens = 1;       // tokens per routing workgroup or unit
+constexpr int kSelectTokensBatch = 4;  // of the single launch's batch form: one per wavefront
 
 
-// LDS of one token's routing.
+// LDS of the routing of ST tokens.
+template <int ST>
 struct SelectLds {
-  float logit[kSelectTokens][kMaxExperts];
-  float choice[kSelectTokens][kMaxExperts];
-  unsigned long long key[kSelectTokens][kMaxExperts];  // VPL >= 8: keys of lane l at [64j + l]
+  float logit[ST][kMaxExperts];
+  float choice[ST][kMaxExperts];
+  unsigned long long key[ST][kMaxExperts];  // VPL >= 8: keys of lane l at [64j + l]
   float bias[kMaxExperts];                             // the router bias (sigmoid gate)
-  float gscore[kSelectTokens][kMaxGroups];
-  int pick_id[kSelectTokens][kMaxTopK];
-  float pick_val[kSelectTokens][kMaxTopK];
+  float gscore[ST][kMaxGroups];
+  int pick_id[ST][kMaxTopK];
+  float pick_val[ST][kMaxTopK];
 };
 
 // The gate's probability of a logit (sigmoid), or the logit itself (softmax, whose weights
@@ -715,6 +778,19 @@ __device__ __forceinline__ float gate_prob(float logit, int gate) {
   return gate == MEGAMOE_GATE_SIGMOID ? 1.0f / (1.0f + expf(-logit)) : logit;
 }
 
+// The batch form's permutation, written as the tokens are routed: slot (t, k)'s row within its
+// expert is the count of the expert's rows so far (in no fixed order: a row's results do not
+// depend on it), perm[e*T + rank] the entry t*K + k and inv the expert and rank in one word. The
+// permute then only scans the counts, where ranking every entry in one workgroup took 219 us at
+// 2048 tokens x 8 slots. counts is NULL in the other forms.
+constexpr int kRankBits = 21;  // T*K < 2^21 and E <= 1024 (validate)
+struct TokenRanks {
+  int* counts;  // [E], zero when the call starts
+  int* perm;    // [E, T]
+  int* inv;     // [T*K]
+  int T;
+};
+
 // Wavefront `wv` routes token t from the logits in LDS (one wavefront per token, no barrier).
 // The logits and the choices stay in LDS and are read again where needed (a probability is
 // recomputed from its logit by the same expression, so it has the same bits). The selection
@@ -722,11 +798,11 @@ __device__ __forceinline__ float gate_prob(float logit, int gate) {
 // they go to LDS and the lane keeps only its largest: with 8 or 16 keys of 64 bits per lane
 // held in registers, the single-launch kernel, whose register budget the expert units set,
 // spilled them to scratch.
-template <int VPL, bool CO>
-__device__ __forceinline__ void route_token(SelectLds& L, int lane, int wv, int t, bool token_ok, int E, int K,
+template <int VPL, bool CO, int ST>
+__device__ __forceinline__ void route_token(SelectLds<ST>& L, int lane, int wv, int t, bool token_ok, int E, int K,
                                             int G, int TG, int gate,
                                             int renorm, float scaling, int64_t* __restrict__ ids_out,
-                                            float* __restrict__ w_out) {
+                                            float* __restrict__ w_out, const TokenRanks& ranks) {
   const float* logit_lds = L.logit[wv];
   float* choice_lds = L.choice[wv];
   auto& gscore = L.gscore;
@@ -878,21 +954,26 @@ __device__ __forceinline__ void route_token(SelectLds& L, int lane, int wv, int 
   if (lane < K) {
     store_out<CO>(&ids_out[(size_t)t * K + lane], (int64_t)my_id);
     store_out<CO>(&w_out[(size_t)t * K + lane], w);
+    if (ranks.counts) {
+      const int rank = __hip_atomic_fetch_add(&ranks.counts[my_id], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      store_out<CO>(&ranks.perm[(size_t)my_id * ranks.T + rank], t * K + lane);
+      store_out<CO>(&ranks.inv[(size_t)t * K + lane], (int)((uint32_t)my_id << kRankBits | (uint32_t)rank));
+    }
   }
 }
 
-// Routing of token `token` (kSelectTokens = 1) by the workgroup's 256 threads: all load and
-// sum the split partials, wavefront 0 routes. ids and weights go out as device-coherent
+// Routing of tokens ST*unit .. +ST-1 by the workgroup's 256 threads: all load and sum the split
+// partials, then a wavefront routes each. ids and weights go out as device-coherent
 // stores (a later workgroup of the single-launch kernel reads them).
-template <int VPL, bool CO>
+template <int VPL, bool CO, int ST>
 __device__ __forceinline__ void select_token(const double* __restrict__ partial, int nsplit,
                                              const float* __restrict__ logits_in, const float* __restrict__ bias,
                                              int T, int E, int K, int G, int TG, int gate, int renorm, float scaling,
-                                             int64_t* __restrict__ ids_out, float* __restrict__ w_out, int token,
-                                             SelectLds& L) {
+                                             int64_t* __restrict__ ids_out, float* __restrict__ w_out, int unit,
+                                             SelectLds<ST>& L, const TokenRanks& ranks) {
   auto& lds_logit = L.logit;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int t0 = token * kSelectTokens, t = t0 + wv;
+  const int t0 = unit * ST, t = t0 + wv;
   const bool token_ok = t < T;
 
   // The bias into LDS (thread i: entries i, i+256, ...), loaded beside the logits' loads.
@@ -902,12 +983,12 @@ __device__ __forceinline__ void select_token(const double* __restrict__ partial,
   for (int r = 0; r < NB; ++r) bias_e[r] = bias ? bias[min((int)threadIdx.x + 256 * r, E - 1)] : 0.0f;
 
   // Logits of the workgroup's tokens into LDS: thread i sums the splits (in split order)
-  // of entries i, i+256, ... (kSelectTokens * E <= 64 * VPL of them, up to kMaxSplits
+  // of entries i, i+256, ... (ST * E <= 64 * VPL of them, up to kMaxSplits
   // splits each), every load issued before the first add.
-  const int n_here = min(kSelectTokens, T - t0) * E;
+  const int n_here = min(ST, T - t0) * E;
   if (logits_in) {
 #pragma unroll
-    for (int r = 0; r < (kSelectTokens * 64 * VPL + 255) / 256; ++r) {
+    for (int r = 0; r < (ST * 64 * VPL + 255) / 256; ++r) {
       const int i = threadIdx.x + 256 * r;
       const float v = logits_in[(size_t)t0 * E + min(i, n_here - 1)];
       if (i < n_here) lds_logit[i / E][i % E] = v;
@@ -915,7 +996,7 @@ __device__ __forceinline__ void select_token(const double* __restrict__ partial,
   } else {
     const size_t stride = (size_t)T * E;
     const double* p = partial + (size_t)t0 * E;
-    constexpr int NE = (kSelectTokens * 64 * VPL + 255) / 256;  // entries per thread
+    constexpr int NE = (ST * 64 * VPL + 255) / 256;  // entries per thread
     constexpr int R = NE < 2 ? NE : 2;                           // entries per round of loads
 #pragma unroll
     for (int r0 = 0; r0 < NE; r0 += R) {
@@ -962,8 +1043,8 @@ __device__ __forceinline__ void select_token(const double* __restrict__ partial,
   __syncthreads();
   // The lane behind an empty asm: the experts' indices derived from it are computed here, not
   // hoisted out of the single-launch kernel's persistent loop and held (or spilled) across it.
-  if (wv < kSelectTokens) route_token<VPL, CO>(L, opaque_lane(), wv, t, token_ok, E, K, G, TG, gate, renorm, scaling,
-                                           ids_out, w_out);
+  if (wv < ST) route_token<VPL, CO, ST>(L, opaque_lane(), wv, t, token_ok, E, K, G, TG, gate, renorm, scaling,
+                                           ids_out, w_out, ranks);
 }
 
 template <int VPL>
@@ -977,9 +1058,9 @@ __global__ __launch_bounds__(256) void k_select(const double* __restrict__ parti
     quant_x_group((int)blockIdx.x - n_sel, x, xq, xs, T, H, pow2);
     return;
   }
-  __shared__ SelectLds lds;
-  select_token<VPL, false>(partial, nsplit, logits_in, bias, T, E, K, G, TG, gate, renorm, scaling, ids_out, w_out,
-                           blockIdx.x, lds);
+  __shared__ SelectLds<kSelectTokens> lds;
+  select_token<VPL, false, kSelectTokens>(partial, nsplit, logits_in, bias, T, E, K, G, TG, gate, renorm, scaling,
+                                          ids_out, w_out, blockIdx.x, lds, TokenRanks{});
 }
 
 
@@ -1148,11 +1229,13 @@ __device__ __forceinline__ void touch_lines(const uint8_t* m0, const uint8_t* m1
 //     expert across tiles (32 + E + E*tile_waves ints). Repeated ids within a token are
 //     found by comparing each entry with its token's other slots.
 // flags[0..1] are two more LDS ints.
-template <bool CO>
+// COUNTED: the entries were ranked as their tokens were routed (TokenRanks); `counted` holds the
+// experts' counts, and a routed chunk's .w its first row within the expert.
+template <bool CO, bool COUNTED = false>
 __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, int64_t base, int T, int K, int E,
                                               int S, int nbI, int nbH, int ks, int chunk, int wide,
                                               const PermuteOut& out, int* smem, int* flags, int tile_waves = 0,
-                                              bool prefix = false) {
+                                              bool prefix = false, const int* counted = nullptr) {
   int* bad = flags;
   int* hits = flags + 1;
   unsigned long long* tmp = (unsigned long long*)smem;  // 16
@@ -1160,8 +1243,9 @@ __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, i
   unsigned* bm = (unsigned*)(cnt + E);                   // E * words (bitmap), or tile_waves * E (tiles)
   const int words = (T + 31) / 32;
   const int tid = threadIdx.x, nt = blockDim.x, n = T * K;
-  for (int i = tid; i < E; i += nt) cnt[i] = 0;
-  if (!tile_waves)
+  for (int i = tid; i < E; i += nt)
+    cnt[i] = COUNTED ? __hip_atomic_load(&counted[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+  if (!COUNTED && !tile_waves)
     for (int i = tid; i < E * words; i += nt) bm[i] = 0u;
   if (tid == 0) {
     *bad = 0;
@@ -1174,7 +1258,7 @@ __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, i
   int keep[kKeep];
 #pragma unroll
   for (int j = 0; j < kKeep; ++j) keep[j] = 0;
-  for (int i = tid, j = 0; i < n; i += nt, ++j) {
+  for (int i = tid, j = 0; !COUNTED && i < n; i += nt, ++j) {
     const int64_t e64 = ids[i] - base;
     const int t = i / K;
 #pragma unroll
@@ -1268,19 +1352,19 @@ __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, i
       }
     } else {
       for (int i = 0; i < a4; ++i) {
-        const int4 ch = make_int4(e, off + chunk * i, min(chunk, c - chunk * i), 0);
+        const int4 ch = make_int4(e, off + chunk * i, min(chunk, c - chunk * i), COUNTED ? chunk * i : 0);
         store_out<CO>(&out.gu[gbase[0] + gshared[0] + p4 + i], ch);
         store_out<CO>(&out.dn[dbase[0] + dshared[0] + p4 + i], ch);
         store_out<CO>(&out.dn_of_gu[gbase[0] + gshared[0] + p4 + i], dbase[0] + dshared[0] + p4 + i);
       }
       if (a2) {
-        const int4 ch = make_int4(e, off + chunk * full, rem, 0);
+        const int4 ch = make_int4(e, off + chunk * full, rem, COUNTED ? chunk * full : 0);
         store_out<CO>(&out.gu[gbase[1] + gshared[1] + p2], ch);
         store_out<CO>(&out.dn[dbase[1] + dshared[1] + p2], ch);
         store_out<CO>(&out.dn_of_gu[gbase[1] + gshared[1] + p2], dbase[1] + dshared[1] + p2);
       }
       if (a1) {
-        const int4 ch = make_int4(e, off + chunk * full, rem, 0);
+        const int4 ch = make_int4(e, off + chunk * full, rem, COUNTED ? chunk * full : 0);
         store_out<CO>(&out.gu[gbase[2] + gshared[2] + p1], ch);
         store_out<CO>(&out.dn[dbase[2] + dshared[2] + p1], ch);
         store_out<CO>(&out.dn_of_gu[gbase[2] + gshared[2] + p1], dbase[2] + dshared[2] + p1);
@@ -1327,6 +1411,7 @@ __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, i
   for (int i = tid; i < dtot; i += nt) store_out<CO>(&out.ready[(size_t)i * out.ready_stride], 0);
   if (out.pairs)
     for (int i = tid; i < (S * (s4 + s2 + s1) + t4 + t2 + t1) * nbI; i += nt) store_out<CO>(&out.pairs[i], 0);
+  if constexpr (COUNTED) return;
   __syncthreads();
   if (!tile_waves) {
     // With `prefix` (long rows: the stream-ordered permute of many rows), each expert's row
@@ -2543,7 +2628,7 @@ __device__ __forceinline__ void gateup_batch_unit(const GateUpArgs& a, const uin
 #pragma unroll
   for (int i = 0; i < 4; ++i) op.a[i] = (w & 1 ? wu : wg) + (size_t)(64 * (w >> 1) + 16 * i) * H;
   op.sw = lane & 1 ? su : sg;
-  const auto token = [&cr](int r) { return row_token(cr, r); };
+  const auto token = [&cr](int r) { return cr.perm ? cr.perm[r] / cr.K : cr.row0 + r; };
   batch_rows(op, A16 ? reinterpret_cast<const uint8_t*>(a.x16) : a.xq, (size_t)H * (A16 ? 2 : 1), cr.n, token);
   op.sx = A16 ? nullptr : a.xs + (size_t)token(min(c0 + (lane & (16 * NT - 1)), cr.n - 1)) * nkb;
   f32x4 acc[8][NT];
@@ -2610,7 +2695,7 @@ __device__ __forceinline__ void gateup_batch_work(const GateUpArgs& a, int u, fl
   const int nbI = a.I / kBlock, nkb = a.H / kBlock;
   const int4 ch = a.chunks[u / nbI];
   const bool shared = ch.x == a.E;
-  const int jb = ch.w + u % nbI;
+  const int jb = (shared ? ch.w : 0) + u % nbI;  // a shared copy's first block
   const int rot = (ch.x * nbI + jb) % nkb;
   const uint8_t *wg, *wu;
   const float *sg, *su;
@@ -2640,7 +2725,7 @@ __device__ __forceinline__ void gateup_batch_work(const GateUpArgs& a, int u, fl
     hq = a.hq_r;
     hs = a.hs_r;
     h16 = a.h16_r;
-    perm = a.perm;
+    perm = a.perm + (size_t)ch.x * a.T + ch.w;  // the chunk's entries (TokenRanks)
     ldh = a.I;
   }
   wg += rowblk * kBlock * a.H;
@@ -3072,11 +3157,20 @@ struct SlotRows {
 
 // Where slot s of token t left its d row: row inv[t*K + s] of the grouped rows, or in the
 // dense schedule (dense_t = T > 0) row ids[t*K + s] * T + t, its expert's row of the token.
+// With `offsets` (the batch form), inv holds the expert and the rank within it (TokenRanks).
 struct SlotMap {
   const int* inv;
   const int64_t* ids;
   int dense_t;
+  const int* offsets = nullptr;
 };
+
+// The batch form's slot rows from the expert and rank that inv holds.
+__device__ __forceinline__ void place_slots(const SlotMap& m, SlotRows& r) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    r.row[u] = m.offsets[(uint32_t)r.row[u] >> kRankBits] + (r.row[u] & ((1 << kRankBits) - 1));
+}
 
 __device__ __forceinline__ void load_slots(const SlotMap& m, const float* __restrict__ wts, int K, int t, int s0,
                                            SlotRows& r) {
@@ -3086,6 +3180,7 @@ __device__ __forceinline__ void load_slots(const SlotMap& m, const float* __rest
   } else {
 #pragma unroll
     for (int u = 0; u < 8; ++u) r.row[u] = m.inv[t * K + min(s0 + u, K - 1)];  // clamped, unconditional loads
+    if (m.offsets) place_slots(m, r);
   }
 #pragma unroll
   for (int u = 0; u < 8; ++u)
@@ -3414,6 +3509,7 @@ struct LayerArgs {
                       // of this kernel's own, zeroed by the last workgroup of each call
   int n_ready;        // dense: readiness counters to zero at the end (down chunks)
   int pad_;
+  TokenRanks ranks;   // the batch form's permutation (counts NULL: none)
 };
 
 __device__ __forceinline__ int* signal_flag(int* ctl, int sig, int line) {
@@ -3457,19 +3553,20 @@ __device__ __forceinline__ int publish_count(int* ctl, int word, int add, int ne
   return old;
 }
 
-template <int NTT>
+template <int NTT, bool PIPE>
 __device__ __forceinline__ void layer_router(const LayerArgs& a, int unit, uint8_t* lds) {
-  router_tile<NTT, true>(a.x, a.router, a.partial, a.T, a.H, a.E, a.n_et, a.nsplit, unit,
+  router_tile<NTT, true, PIPE>(a.x, a.router, a.partial, a.T, a.H, a.E, a.n_et, a.nsplit, unit,
                          reinterpret_cast<f64x4*>(lds));
 }
 
+template <bool PIPE>
 __device__ __forceinline__ void layer_router_unit(const LayerArgs& a, int r, uint8_t* lds) {
   if (a.ntt == 1)
-    layer_router<1>(a, r, lds);
+    layer_router<1, PIPE>(a, r, lds);
   else if (a.ntt == 2)
-    layer_router<2>(a, r, lds);
+    layer_router<2, PIPE>(a, r, lds);
   else
-    layer_router<4>(a, r, lds);
+    layer_router<4, PIPE>(a, r, lds);
 }
 
 // A routing unit waits this long for the router signal before it looks for router units
@@ -3515,21 +3612,25 @@ __device__ __forceinline__ int rescue_router_unit(int n_first, int* ctl, int* ld
   }
 }
 
-template <int VPL>
-__device__ __forceinline__ void layer_select(const LayerArgs& a, int token, uint8_t* lds) {
-  select_token<VPL, true>(a.partial, a.nsplit, nullptr, a.bias, a.T, a.E, a.K, a.G, a.TG, a.gate, a.renorm, a.scaling,
-                    a.ids, a.wts, token, *reinterpret_cast<SelectLds*>(lds));
+template <int VPL, int ST>
+__device__ __forceinline__ void layer_select(const LayerArgs& a, int unit, uint8_t* lds) {
+  select_token<VPL, true, ST>(a.partial, a.nsplit, nullptr, a.bias, a.T, a.E, a.K, a.G, a.TG, a.gate, a.renorm,
+                              a.scaling, a.ids, a.wts, unit, *reinterpret_cast<SelectLds<ST>*>(lds),
+                              ST == kSelectTokens ? TokenRanks{} : a.ranks);
 }
 
 // Where the combine finds each slot's d row: the permute's inverse, or in the dense schedule
 // the row of the slot's expert for the token.
+template <bool BATCH>
 __device__ __forceinline__ SlotMap layer_slots(const LayerArgs& a) {
+  if constexpr (BATCH) return SlotMap{a.po.inv, nullptr, 0, a.po.offsets};
   return a.dense ? SlotMap{nullptr, a.ids, a.T} : SlotMap{a.po.inv, nullptr, 0};
 }
 
 // Combine unit c: outputs [c * kCombineUnit, +kCombineUnit) of y, as k_combine (with
 // `use_first`, `first` holds the thread's first eight slots, loaded already). The slots pass by
 // value: behind a pointer that may be null they were kept in scratch memory.
+template <bool BATCH>
 __device__ __forceinline__ void layer_combine(const LayerArgs& a, int c, const SlotRows& first, bool use_first) {
   const DownArgs& dn = a.ex.dn;
   const int i = c * (kCombineUnit / 8) + threadIdx.x, per_row = a.H / 8;
@@ -3540,7 +3641,7 @@ __device__ __forceinline__ void layer_combine(const LayerArgs& a, int c, const S
   }
   const int t = i / per_row, h0 = (i % per_row) * 8;
   float acc[8];
-  const SlotMap m = layer_slots(a);
+  const SlotMap m = layer_slots<BATCH>(a);
   if (a.ks > 1)
     combine8_parts(dn.p_r, dn.p_s, a.ks, m, a.wts, a.T, dn.rows_r, a.H, a.K, a.S, t, h0, acc, first, use_first);
   else
@@ -3612,10 +3713,12 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
   int *flags = misc.flags, *units = misc.units;
   double* part = misc.part;
   static_assert(sizeof(LayerArgs) % 8 == 0 && offsetof(LayerArgs, ex) == 0, "argument segment layout");
-  static_assert(sizeof(SelectLds) <= 4 * kRingWave && (kRouterWaves - 1) * 4 * 64 * sizeof(f64x4) <= 4 * kRingWave,
+  constexpr int ST = BATCH ? kSelectTokensBatch : kSelectTokens;  // tokens per routing unit
+  static_assert(sizeof(SelectLds<ST>) <= (BATCH ? kBatchRing : 4 * kRingWave) && (kRouterWaves - 1) * 4 * 64 * sizeof(f64x4) <= 4 * kRingWave,
                 "front-end scratch in the rings");
   int* ctl = args.ctl;
-  const int fixed = args.n_norm + args.n_router + args.T;  // units listed before the routing is known
+  const int n_sel = (args.T + ST - 1) / ST;                  // routing units
+  const int fixed = args.n_norm + args.n_router + n_sel;  // units listed before the routing is known
   // Router units [0, n_first) go to the workgroup of the same index, the rest through the
   // queue, whose first entry is unit n_first: 512 workgroups claiming their first unit from
   // one counter at once took ~10 us to be served, and the router phase waited for the last.
@@ -3662,7 +3765,7 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
     } else if (u < a.n_norm + a.n_router) {
       if (a.n_norm) wait_signal(ctl, kSigNormed);
       const int r = u - a.n_norm;
-      layer_router_unit(a, r, rings);
+      layer_router_unit<BATCH>(a, r, rings);
       // Counted unless a rescuing workgroup took it first (then that one counts it).
       publish_fence();
       __syncthreads();
@@ -3673,7 +3776,7 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
     } else {
       const int t = u - a.n_norm - a.n_router;
       if (a.n_norm) wait_signal(ctl, kSigNormed);
-      // This token's row of x in E4M3 per 128 (needs nothing else; runs while the router does).
+      // This unit's rows of x in E4M3 per 128 (needs nothing else; runs while the router does).
       const int nbh = a.H / kBlock, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
       const bool back = resume >= 0;  // after a rescued router unit: look again at once
       if (!back) {
@@ -3681,9 +3784,17 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
         // the quantized x holds its bf16 h. A write-through store of x there would leave the
         // line in this XCD's L2, where a down unit on the same XCD, reading the h row that a
         // gate/up unit on another XCD wrote later, would find the stale copy.
-        if constexpr (!A16)
-          quant_row(a.x + (size_t)t * a.H, a.xq + (size_t)t * a.H, a.xs + (size_t)t * nbh, nbh, a.pow2, lane, wv,
+        auto quantize = [&](int r) {
+          quant_row(a.x + (size_t)r * a.H, a.xq + (size_t)r * a.H, a.xs + (size_t)r * nbh, nbh, a.pow2, lane, wv,
                     reinterpret_cast<float*>(rings));
+        };
+        if constexpr (!A16) {
+          if constexpr (ST == 1)
+            quantize(t);
+          else if (t * ST + wv < a.T)
+            quant_row_wave(a.x + (size_t)(t * ST + wv) * a.H, a.xq + (size_t)(t * ST + wv) * a.H,
+                           a.xs + (size_t)(t * ST + wv) * nbh, nbh, a.pow2, lane);
+        }
         // The dense schedule's gate/up units read every token's row once all are quantized
         // (W8A16: once every routing unit has passed its wait for the normalized rows).
         if (a.dense) publish_count(ctl, kCtlQuant, 1, a.T, kSigQuant, &units[0]);
@@ -3704,22 +3815,23 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
       }
       if (!routed) wait_signal(ctl, kSigRouted);
       if (a.vpl == 1)
-        layer_select<1>(a, t, rings);
+        layer_select<1, ST>(a, t, rings);
       else if (a.vpl == 2)
-        layer_select<2>(a, t, rings);
+        layer_select<2, ST>(a, t, rings);
       else if (a.vpl == 4)
-        layer_select<4>(a, t, rings);
+        layer_select<4, ST>(a, t, rings);
       else if (a.vpl == 8)
-        layer_select<8>(a, t, rings);
+        layer_select<8, ST>(a, t, rings);
       else
-        layer_select<16>(a, t, rings);
-      if (publish_count(ctl, kCtlSelected, 1, a.T, -1, &units[0]) == a.T - 1) {
+        layer_select<16, ST>(a, t, rings);
+      if (publish_count(ctl, kCtlSelected, 1, n_sel, -1, &units[0]) == n_sel - 1) {
         // Every token is routed: this workgroup runs the permute, then publishes the lists.
         acquire_after_wait();
-        permute_block<true>(a.ids, 0, a.T, a.K, a.E, a.S, a.ex.gu.I / kBlock, a.H / kBlock / (BATCH ? 2 : 1), a.ks,
-                            BATCH ? kChunkRowsBatch : (A16 ? kChunkRowsA16 : kChunkRows), 0,
-                            a.po, reinterpret_cast<int*>(rings), flags,
-                            permute_tile_waves(a.T, a.E, 256, kPermuteLdsInts));
+        permute_block<true, BATCH>(a.ids, 0, a.T, a.K, a.E, a.S, a.ex.gu.I / kBlock, a.H / kBlock / (BATCH ? 2 : 1),
+                                   a.ks, BATCH ? kChunkRowsBatch : (A16 ? kChunkRowsA16 : kChunkRows), 0, a.po,
+                                   reinterpret_cast<int*>(rings), flags,
+                                   BATCH ? 0 : permute_tile_waves(a.T, a.E, 256, kPermuteLdsInts), false,
+                                   a.ranks.counts);
         publish_fence();
         __syncthreads();
         raise_signal(ctl, kSigPermuted);
@@ -3844,14 +3956,31 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
     SlotRows first;
     {
       const int i = (u - experts_end) * (kCombineUnit / 8) + threadIdx.x, per_row = a.H / 8;
-      load_slots(layer_slots(a), a.wts, a.K, min(i, a.T * per_row - 1) / per_row, 0, first);
+      load_slots(layer_slots<BATCH>(a), a.wts, a.K, min(i, a.T * per_row - 1) / per_row, 0, first);
     }
     if (n_dn) wait_signal(ctl, kSigDown, 1 + a.force_timeout, a.force_timeout ? (uint64_t)2000 : kWaitTicks);
+    if constexpr (BATCH) {
+      // Every workgroup comes here with the down units' end: the units go round the grid (each
+      // workgroup's last claim is a place of its own in it). A unit's slots load two units ahead and
+      // its d rows' places one, so no load waits for another of the same round.
+      const int n_comb = total - experts_end, per_row = a.H / 8, step = (int)gridDim.x;
+      auto token = [&](int c) { return min(c * (kCombineUnit / 8) + (int)threadIdx.x, a.T * per_row - 1) / per_row; };
+      SlotRows ahead;
+      load_slots(SlotMap{a.po.inv, nullptr, 0}, a.wts, a.K, token(u - experts_end + step), 0, ahead);
+      for (int c = u - experts_end; c < n_comb; c += step) {
+        SlotRows next_rows = ahead;
+        place_slots(layer_slots<BATCH>(a), next_rows);
+        load_slots(SlotMap{a.po.inv, nullptr, 0}, a.wts, a.K, token(c + 2 * step), 0, ahead);
+        layer_combine<BATCH>(a, c, first, true);
+        first = next_rows;
+      }
+      u = total;
+    }
     bool use_first = true;
     while (u < total) {
       __syncthreads();
       if (threadIdx.x == 0) next = n_first + claim_ticket(&ctl[kCtlQueue]);
-      layer_combine(a, u - experts_end, first, use_first);
+      layer_combine<BATCH>(a, u - experts_end, first, use_first);
       use_first = false;
       if (threadIdx.x == 0) slot = next;
       __syncthreads();
@@ -3882,6 +4011,9 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int b = i; b < n_first; b += 256)
       __hip_atomic_store(&ctl[kCtlStart + b * kStartStride], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (BATCH)
+      for (int e = i; e < args.E; e += 256)
+        __hip_atomic_store(&args.ranks.counts[e], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int c = i; c < args.n_ready; c += 256)  // the dense schedule's readiness counters
       __hip_atomic_store(&args.ex.ready[(size_t)c * args.ex.ready_stride], 0, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
@@ -5098,7 +5230,8 @@ inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
   size_t xn, partial, xq, xs, counts, offsets, meta, perm, inv, gu, dn, dn_of_gu, ready, ready_l, pairs, hq_r, hs_r,
-      hq_s, hs_s, st_r, st_s, h16_r, h16_s, d_r, d_s, p_r, p_s, spare, ctl, total;
+      hq_s, hs_s, st_r, st_s, h16_r, h16_s, d_r, d_s, p_r, p_s, spare, ctl, eperm, ecounts, total;
+  size_t total_ordered;  // what the stream-ordered form needs
   int nsplit;
   int ks;  // K parts of each down unit
   int ready_stride;  // ints between two readiness counters
@@ -5167,21 +5300,29 @@ bool split_gate_up(const megamoe_desc& d) {
 // activation rows through LDS, one workgroup per CU) or the decode units (16-64 rows, two). The
 // decode units stream weights faster while an expert's rows are few (their waves share nothing);
 // past about 16 rows an expert they are bound by activation loads, and past 64 (W8A16: 32) they
-// stream an expert's weights more than once. One call, decode units -> batch units: DeepSeek-V3's
-// shape at 64 / 256 / 512 tokens 767 -> 788, 1165 -> 1105, 1569 -> 1342 us (W8A16 788 -> 824,
-// 1397 -> 1193, 2209 -> 1555), Mixtral's at 64 / 256 / 512 310 -> 278, 559 -> 386, 908 -> 586,
-// Qwen3-30B-A3B's at 128 / 256 / 512 149 -> 158, 181 -> 176, 231 -> 218. Depends on the geometry
-// only; both give the same bits (the separate gate and up units, whose K rotations differ, keep
-// their geometries).
+// stream an expert's weights more than once. The batch form also routes four tokens a unit, ranks
+// entries as they are routed and cuts the router into fewer splits, where the decode form's
+// front end grows with the tokens (the permute of 2048 x 8 entries in one workgroup: 219 us).
+// One call, decode -> batch: DeepSeek-V3's shape at 64 / 128 / 256 / 512 tokens 767 -> 788, 918 ->
+// 907, 1165 -> 1093, 1569 -> 1276 us (W8A16 788 -> 824, 985 -> 937, 1397 -> 1178, 2209 -> 1495),
+// Kimi-K2's at 128 (2.7 rows an expert) 2106 -> 2114, Mixtral's at 64 / 256 / 512 303 -> 277, 559 ->
+// 388, 908 -> 583; experts of few weights pay more for the one workgroup per CU:
+// Qwen3-30B-A3B's at 128 / 192 / 256 / 2048 149 -> 158, 161 -> 164, 181 -> 170, 754 -> 385. Depends on
+// the geometry only; both give the same bits (the separate gate and up units, whose K rotations
+// differ, keep their geometries).
 bool batch_units(const megamoe_desc& d) {
+  const int64_t entries = (int64_t)d.tokens * d.topk, E = d.experts;
+  const bool large = (int64_t)d.hidden * d.intermediate >= ((int64_t)8 << 20);
   return !dense_experts(d) && d.hidden % (2 * kBlock) == 0 &&
-         (d.tokens >= 256 || (int64_t)d.tokens * d.topk >= (int64_t)16 * d.experts);
+         (d.tokens >= 208 || entries >= 16 * E || (large && d.tokens >= 128 && entries >= 4 * E));
 }
 
 Layout make_layout(const megamoe_desc& d) {
   Layout L{};
   const size_t T = d.tokens, H = d.hidden, E = d.experts, K = d.topk, I = d.intermediate, S = d.shared_experts;
-  L.nsplit = router_splits((int)H);
+  const bool batch = batch_units(d);
+  const int splits = router_splits((int)H);
+  L.nsplit = batch ? router_splits_batch((int)H, (int)E, (int)T) : splits;
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t o = at;
@@ -5189,7 +5330,7 @@ Layout make_layout(const megamoe_desc& d) {
     return o;
   };
   L.xn = take(T * H * 2);  // normalized x of the block form
-  L.partial = take((size_t)L.nsplit * T * E * sizeof(double));
+  L.partial = take((size_t)splits * T * E * sizeof(double));  // the most splits' size, at any T
   L.counts = take(E * sizeof(int));
   L.offsets = take((E + 1) * sizeof(int));
   L.meta = take(kMetaInts * sizeof(int));
@@ -5240,6 +5381,12 @@ Layout make_layout(const megamoe_desc& d) {
   L.p_s = take(L.ks > 1 && S ? L.ks * T * H * sizeof(float) : 0);
   L.spare = take(16 * (H > I * (S > 1 ? S : 1) ? H : I * (S > 1 ? S : 1)));
   L.ctl = take(kCtlInts * sizeof(int));  // the single-launch kernel's control words
+  L.total_ordered = at;
+  // The batch form's permutation (TokenRanks): entries by expert behind the fewer partials that its
+  // router leaves, where they fit; the experts' counts among the words that each call leaves zero.
+  const size_t partials = align_up((size_t)L.nsplit * T * E * sizeof(double)), entries = batch ? E * T * sizeof(int) : 0;
+  L.eperm = partials + entries <= align_up((size_t)splits * T * E * sizeof(double)) ? L.partial + partials : take(entries);
+  L.ecounts = take(batch ? E * sizeof(int) : 0);
   L.total = at;
   return L;
 }
@@ -5471,7 +5618,7 @@ int forward_impl(const megamoe_desc* desc, const megamoe_tensors* t, hipStream_t
                                !t->shared_up_scale || !t->shared_down || !t->shared_down_scale))
     return MEGAMOE_ERR_INVALID_ARGUMENT;
   const Layout L = make_layout(d);
-  if (t->workspace_bytes < L.total) return MEGAMOE_ERR_WORKSPACE;
+  if (t->workspace_bytes < L.total_ordered) return MEGAMOE_ERR_WORKSPACE;
   DeviceInfo di;
   if ((rc = device_info(&di))) return rc;
   char* ws = (char*)t->workspace;
@@ -5606,6 +5753,10 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   const size_t units_max = (size_t)la.n_norm + la.n_router + T +
                            expert_units_max(d, L, split, a16 ? kChunkRowsA16 : kChunkRows) +
                            ((size_t)T * H + kCombineUnit - 1) / kCombineUnit;
+  if (batch) {
+    la.ranks = TokenRanks{(int*)(ws + L.ecounts), (int*)(ws + L.eperm), la.po.inv, T};
+    la.ex.gu.perm = la.ranks.perm;
+  }
   la.dense = L.dense;
   la.n_ready = L.n_ready_l;
   if (L.dense) la.ex.ready = (int*)(ws + L.ready_l);
@@ -6182,7 +6333,7 @@ int megamoe_forward_noalloc(const megamoe_desc* desc, const megamoe_tensors* t, 
   int rc = validate(desc);
   if (rc) return rc;
   if (!t) return MEGAMOE_ERR_INVALID_ARGUMENT;
-  if (make_layout(*desc).total > (size_t)MEGAMOE_SCRATCH_BYTES) return MEGAMOE_ERR_SCRATCH;
+  if (make_layout(*desc).total_ordered > (size_t)MEGAMOE_SCRATCH_BYTES) return MEGAMOE_ERR_SCRATCH;
   void* ws = nullptr;
   if ((rc = scratch_address(&ws))) return rc;
   megamoe_tensors with_scratch = *t;
