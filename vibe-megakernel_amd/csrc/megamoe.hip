@@ -1157,6 +1157,7 @@ struct PermuteOut {
   int ready_stride = 1;  // ints between two chunks' counters
   int* xcd = nullptr;    // the batch form's per-XCD queues (kXcdInts; NULL: none)
   int ready_min = 0;     // readiness counters zeroed at least (the dense schedule's down chunks)
+  int pairs_min = 0;     // block counters zeroed at least (its gate/up blocks)
 };
 
 // The batch form's work split over the XCDs (the lists in expert order, `wide` 2): XCD x
@@ -1410,7 +1411,8 @@ __device__ __forceinline__ void permute_block(const int64_t* __restrict__ ids, i
   const int dtot = max(s4 + s2 + s1 + t4 + t2 + t1, out.ready_min);
   for (int i = tid; i < dtot; i += nt) store_out<CO>(&out.ready[(size_t)i * out.ready_stride], 0);
   if (out.pairs)
-    for (int i = tid; i < (S * (s4 + s2 + s1) + t4 + t2 + t1) * nbI; i += nt) store_out<CO>(&out.pairs[i], 0);
+    for (int i = tid; i < max((S * (s4 + s2 + s1) + t4 + t2 + t1) * nbI, out.pairs_min); i += nt)
+      store_out<CO>(&out.pairs[i], 0);
   if constexpr (COUNTED) return;
   __syncthreads();
   if (!tile_waves) {
@@ -2387,7 +2389,7 @@ struct GateUpArgs {
   int swiglu;                   // 0: fp32 product rounded once; 1: bf16 silu, bf16 product
   float limit;                  // > 0: SwiGLU clamp (gate above, up both sides)
   int dense;                    // the dense schedule: units from dense_gu_chunk, h rows e*T + t
-  int pad_;
+  int parts;                    // the small form: units per 128-row block (2, 4 or 8)
   const uint16_t* x16;          // W8A16: the bf16 rows [T, H] the experts read (x, or the normalized x)
   uint16_t* h16_r;              // W8A16: bf16 h of the routed rows [rows_r, I]
   uint16_t* h16_s;              // W8A16: of the shared rows [T, S*I]
@@ -2739,6 +2741,145 @@ __device__ __forceinline__ void gateup_batch_work(const GateUpArgs& a, int u, fl
     gateup_batch_unit<2, A16>(a, wg, wu, sg, su, cr, jb, hq, hs, h16, ldh, rot, red, ring, ready);
   else
     gateup_batch_unit<4, A16>(a, wg, wu, sg, su, cr, jb, hq, hs, h16, ldh, rot, red, ring, ready);
+}
+
+// The small form (T <= 16, host: small_parts_wanted): a 128-row block of gate and up worked as P = 2, 4 or 8
+// units of 128/P rows of each, so that a call that hits few experts still spreads its weights
+// evenly over the chip (one user's DeepSeek-V3-shaped call has 144 blocks of 1.8 MB for 256 CUs, and
+// a CU takes in ~29 KB/us however many of its workgroups ask). The four waves work 4/KP pairs of a
+// 16-row gate and a 16-row up tile, each pair over KP = P/2 parts of the K blocks, whose sums are
+// added in part order through LDS. One call of the layer, with down_splits' longer parts: DeepSeek-V3's
+// shape, one token, W8A16 block 169 -> 108 us; Qwen3-30B-A3B's, one token, 50 -> 40; Mixtral's, five
+// tokens, 235 -> 222.
+//
+// W8A16: h goes out as it is, and every unit counts towards the chunk's readiness. W8A8: h goes to
+// staging rows in bf16; the unit that finishes its block last requantizes the block's rows (per
+// 128, as the whole-block units) and alone counts. Staged lines are written once and read by that
+// unit after the block's counter has shown every writer done. In the dense schedule units of one
+// block may have worked every token or, once the routing was known, the routed rows: the last
+// unit takes the routed rows if it is known by then (every unit wrote those), else all tokens (no
+// unit can have known). `known_now` says so: dense_state for the unit's expert.
+//
+// Returns whether the unit (its block) counts.
+template <bool A16, class F>
+__device__ __forceinline__ bool gateup_small_work(const GateUpArgs& a, int u, f32x4 (*part)[2][64], int* flag,
+                                                  uint8_t* ring, const ReadyWait& ready, bool known, F&& known_now) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nbI = a.I / kBlock, H = a.H, nkb = H / kBlock, P = a.parts, KP = P / 2;
+  const int b = u / P, pt = u % P;
+  const int4 ch = a.dense ? dense_gu_chunk(b / nbI, a.E, a.S, a.T, nbI) : a.chunks[b / nbI];
+  const int jb = ch.w + b % nbI;
+  const int pr = KP == 1 ? w : (KP == 2 ? w >> 1 : 0), kp = KP == 1 ? 0 : (KP == 2 ? w & 1 : w);
+  const int nkp = nkb / KP, row0 = pt * (kBlock / P) + 16 * pr;
+  const uint8_t *wg, *wu;
+  const float *sg, *su;
+  uint8_t* hq;
+  float* hs;
+  uint16_t* h16;
+  int ldh;
+  ChunkRows cr;
+  if (ch.x == a.E) {
+    wg = a.sgate + (size_t)jb * kBlock * H;
+    wu = a.sup + (size_t)jb * kBlock * H;
+    sg = a.sgate_scale + (size_t)jb * nkb;
+    su = a.sup_scale + (size_t)jb * nkb;
+    cr = ChunkRows{ch.z, ch.y, nullptr, a.K};
+    hq = a.hq_s;
+    hs = a.hs_s;
+    h16 = A16 ? a.h16_s : a.st_s;
+    ldh = a.S * a.I;
+  } else {
+    const size_t rowblk = (size_t)ch.x * nbI + jb;
+    wg = a.gate + rowblk * kBlock * H;
+    wu = a.up + rowblk * kBlock * H;
+    sg = a.gate_scale + rowblk * nkb;
+    su = a.up_scale + rowblk * nkb;
+    cr = !a.dense ? ChunkRows{ch.z, ch.y, a.perm, a.K}
+                  : (known ? routed_rows(ch.x, a.T, a.K, a.offsets, a.perm) : dense_rows(ch.x, a.T, a.K));
+    hq = a.hq_r;
+    hs = a.hs_r;
+    h16 = A16 ? a.h16_r : a.st_r;
+    ldh = a.I;
+  }
+  Operands<2, 1, 2> op;
+  op.lda = H;
+  op.spare = a.spare;
+  op.a[0] = wg + (size_t)row0 * H + (size_t)kp * nkp * kBlock;
+  op.a[1] = wu + (size_t)row0 * H + (size_t)kp * nkp * kBlock;
+  op.sw[0] = sg + kp * nkp;
+  op.sw[1] = su + kp * nkp;
+  const int tok = row_token(cr, min(lane & 15, cr.n - 1));
+  if constexpr (A16) {
+    op.b[0] = reinterpret_cast<const uint8_t*>(a.x16 + (size_t)tok * H) + (size_t)kp * nkp * 2 * kBlock + 32 * (lane >> 4);
+    op.sx[0] = nullptr;
+  } else {
+    op.b[0] = a.xq + (size_t)tok * H + (size_t)kp * nkp * kBlock + 16 * (lane >> 4);
+    op.sx[0] = a.xs + (size_t)tok * nkb + kp * nkp;
+  }
+  f32x4 acc[2][1];
+  stream_gemm<2, 1, 2, 4, A16>(op, nkp, (ch.x * nbI + jb + pt) % nkp, ring, acc, ready);
+  if (KP > 1) {
+    if (kp > 0) {
+      part[pr * (KP - 1) + kp - 1][0][lane] = acc[0][0];
+      part[pr * (KP - 1) + kp - 1][1][lane] = acc[1][0];
+    }
+    __syncthreads();
+    if (kp == 0)
+      for (int q = 0; q < KP - 1; ++q)
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const f32x4 o = part[pr * (KP - 1) + q][r][lane];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[r][0][v] = __fadd_rn(acc[r][0][v], o[v]);
+        }
+  }
+  if (kp == 0 && (lane & 15) < cr.n) {
+    const bool bf16_silu = a.swiglu != 0;
+    const float L = a.limit > 0.0f ? a.limit : INFINITY;
+    uint32_t bits[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) bits[v] = __float_as_uint(swiglu_h(acc[0][0][v], acc[1][0][v], L, bf16_silu)) >> 16;
+    const int orow = cr.by_token ? cr.out_base + tok : cr.row0 + (lane & 15);
+    uint16_t* dst = h16 + (size_t)orow * ldh + (size_t)jb * kBlock + row0 + 4 * (lane >> 4);
+    store_coherent(reinterpret_cast<uint64_t*>(dst),
+                   (uint64_t)(bits[0] | (bits[1] << 16)) | ((uint64_t)(bits[2] | (bits[3] << 16)) << 32));
+  }
+  if constexpr (A16) return true;
+  publish_fence();
+  __syncthreads();
+  if (threadIdx.x == 0) *flag = atomicAdd(&a.pairs[b], 1) == P - 1;
+  __syncthreads();
+  if (!*flag) return false;
+  acquire_after_wait();
+  if (cr.by_token && !known) {
+    const int st = known_now();
+    if (st == 2) return true;  // no token picked the expert: no combine reads its rows
+    if (st == 1) cr = routed_rows(ch.x, a.T, a.K, a.offsets, a.perm);
+  }
+  const int nbh = scale_ld(ldh / kBlock), l = lane & 31;
+  for (int r0 = 0; r0 < cr.n; r0 += 8) {  // a half wavefront per row
+    const int r = r0 + 2 * w + (lane >> 5);
+    const size_t orow = (size_t)out_row(cr, min(r, cr.n - 1));
+    const uint2 four = *reinterpret_cast<const uint2*>(h16 + orow * ldh + (size_t)jb * kBlock + 4 * l);
+    const float s = act_scale(__uint_as_float(half_wave_max_u32(bf16x4_absmax_bits(four)) << 16), a.pow2);
+    const uint32_t q = e4m3x4(clamp448(bf16_bits_to_f32(four.x & 0xffffu) / s), clamp448(bf16_bits_to_f32(four.x >> 16) / s),
+                              clamp448(bf16_bits_to_f32(four.y & 0xffffu) / s), clamp448(bf16_bits_to_f32(four.y >> 16) / s));
+    if (r < cr.n) {
+      store_coherent(reinterpret_cast<uint32_t*>(hq + orow * ldh + (size_t)jb * kBlock + 4 * l), q);
+      if (l == 0) store_coherent(hs + orow * nbh + jb, s);
+    }
+  }
+  return true;
+}
+
+// A small-form unit that the dense schedule skips (no token picked its expert): it counts in its
+// block all the same. Returns whether the block is now complete.
+template <bool A16>
+__device__ __forceinline__ bool skip_small_unit(const GateUpArgs& a, int u, int* flag) {
+  if constexpr (A16) return true;
+  if (threadIdx.x == 0) *flag = atomicAdd(&a.pairs[u / a.parts], 1) == a.parts - 1;
+  __syncthreads();
+  return *flag != 0;
 }
 
 // One half of a gate/up block: rows [jb*128, jb*128+128) of gate (half 0) or of up (half 1)
@@ -3358,19 +3499,22 @@ struct ExpertArgs {
 // (gateup_unit). The two give the same bits; the host picks one from the geometry.
 // A16: the W8A16 form (bf16 activations and h; whole-block gate/up units, chunks of at most
 // 32 rows).
-template <bool SPLIT, bool A16 = false>
-__global__ __launch_bounds__(256, 2) void k_experts(ExpertArgs args) {
+// SMALL: the small form (gateup_small_work).
+template <bool SPLIT, bool A16, bool SMALL>
+__device__ __forceinline__ void experts_body(const ExpertArgs& args) {
   typedef const __attribute__((address_space(4))) ExpertArgs* ArgsPtr;
   __shared__ float red[4][64];
   __shared__ __attribute__((aligned(16))) uint8_t rings[4 * kRingWave];  // one weight ring per wavefront
   __shared__ int slot, flag;
+  __shared__ f32x4 part[3][2][64];  // small form: sums of the K parts
   static_assert(sizeof(ExpertArgs) % 8 == 0, "argument segment layout");
   int* meta = args.gu.meta;
   // The dense schedule's lists come from the geometry (the permute has run: its counts say
   // which experts no token picked, and their units are skipped).
   const bool dense = args.gu.dense != 0;
   const int nbI0 = args.gu.I / kBlock, sh = args.gu.S > 0 ? 1 : 0;
-  const int total_gu = dense ? (args.gu.S + args.gu.E) * nbI0 : (SPLIT ? 2 : 1) * meta[kMetaUnitsGU];
+  const int per = SPLIT ? 2 : (SMALL ? args.gu.parts : 1);  // units per 128-row block of gate/up
+  const int total_gu = per * (dense ? (args.gu.S + args.gu.E) * nbI0 : meta[kMetaUnitsGU]);
   const int total = total_gu + (dense ? (args.gu.E + sh) * (args.dn.H / kBlock) * args.dn.ks : meta[kMetaUnitsDN]);
   // Every unit, the first included, is claimed from the queue: a unit that a down unit
   // waits for is then always held by a running workgroup (one that has not started yet
@@ -3400,6 +3544,14 @@ __global__ __launch_bounds__(256, 2) void k_experts(ExpertArgs args) {
       if constexpr (SPLIT) {
         done = gateup_work_split(a.gu, u, red, &flag, ring,
                                  claiming(ReadyWait{nullptr, 0, nullptr}, &meta[kMetaQueueGU], &ticket));
+      } else if constexpr (SMALL) {
+        const int c = u / per / nbI;
+        if (dense && c >= a.gu.S && a.gu.offsets[c - a.gu.S + 1] == a.gu.offsets[c - a.gu.S])
+          done = skip_small_unit<A16>(a.gu, u, &flag);
+        else
+          done = gateup_small_work<A16>(a.gu, u, part, &flag, ring,
+                                        claiming(ReadyWait{nullptr, 0, nullptr}, &meta[kMetaQueueGU], &ticket), true,
+                                        [] { return 1; });
       } else {
         const int c = u / nbI;
         if (!(dense && c >= a.gu.S && a.gu.offsets[c - a.gu.S + 1] == a.gu.offsets[c - a.gu.S]))
@@ -3409,13 +3561,14 @@ __global__ __launch_bounds__(256, 2) void k_experts(ExpertArgs args) {
       if (done) {
         publish_fence();
         __syncthreads();
-        const int dc = dense ? dense_dn_of_gu(u / nbI, a.gu.S) : a.dn_of_gu[(SPLIT ? u >> 1 : u) / nbI];
+        const int dc = dense ? dense_dn_of_gu(u / per / nbI, a.gu.S) : a.dn_of_gu[u / per / nbI];
         if (threadIdx.x == 0) atomicAdd(&a.ready[(size_t)dc * a.ready_stride], 1);
       }
     } else {
       const int v = u - total_gu, c = v / (nbH * a.dn.ks), e = c - (a.dn.S > 0 ? 1 : 0);
       if (!(dense && e >= 0 && a.gu.offsets[e + 1] == a.gu.offsets[e])) {
-        const int need = dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI);
+        const int need = (SMALL && A16 ? per : 1) *
+                         (dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI));
         down_work<false, A16>(a.dn, v,
                               claiming(ReadyWait{&a.ready[(size_t)c * a.ready_stride], need, &meta[kMetaError]},
                                        &meta[kMetaQueueGU], &ticket),
@@ -3426,6 +3579,16 @@ __global__ __launch_bounds__(256, 2) void k_experts(ExpertArgs args) {
     __syncthreads();
     u = slot;
   }
+}
+
+template <bool SPLIT, bool A16 = false>
+__global__ __launch_bounds__(256, 2) void k_experts(ExpertArgs args) {
+  experts_body<SPLIT, A16, false>(args);
+}
+
+template <bool A16>
+__global__ __launch_bounds__(256, 2) void k_experts_small(ExpertArgs args) {
+  experts_body<false, A16, true>(args);
 }
 
 // =======================================================================================
@@ -3508,7 +3671,7 @@ struct LayerArgs {
   int dense;          // the dense schedule (host: dense_experts); ex.ready then points at counters
                       // of this kernel's own, zeroed by the last workgroup of each call
   int n_ready;        // dense: readiness counters to zero at the end (down chunks)
-  int pad_;
+  int n_pairs;        // dense small form: block counters to zero at the end
   TokenRanks ranks;   // the batch form's permutation (counts NULL: none)
 };
 
@@ -3701,13 +3864,15 @@ struct LayerMisc {
 
 // A16: the W8A16 form (bf16 activations into the expert units, chunks of at most 32 rows).
 // BATCH: the batch units (gateup_batch_work, down_batch_work).
-template <bool SPLIT, bool A16, bool BATCH>
+// SMALL: the small form (gateup_small_work).
+template <bool SPLIT, bool A16, bool BATCH, bool SMALL>
 __device__ __forceinline__ void layer_body(const LayerArgs& args) {
   typedef const __attribute__((address_space(4))) LayerArgs* ArgsPtr;
   typedef const __attribute__((address_space(4))) ExpertArgs* ExArgsPtr;
   // Weight rings, in the batch form the slots of whole stages; front-end scratch.
   __shared__ __attribute__((aligned(16))) uint8_t rings[BATCH ? kBatchRing + kBatchScales : 4 * kRingWave];
   __shared__ LayerMisc misc;
+  __shared__ f32x4 part_sums[3][2][64];  // small form: sums of the K parts
   float(*red)[64] = misc.red;
   int &slot = misc.slot, &flag = misc.flag;
   int *flags = misc.flags, *units = misc.units;
@@ -3861,14 +4026,15 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
     if (args.ex.gu.S > 0) touch_shared_weights(args.ex, blockIdx.x, gridDim.x);
     wait_ready(ReadyWait{my_signal_flag(ctl, kSigPermuted), 1, &ctl[kCtlError], kWaitTicks, true, 8});
   }
+  const int per = SPLIT ? 2 : (SMALL ? args.ex.gu.parts : 1);  // units per 128-row block of gate/up
   if (threadIdx.x == 0) {
     const int nbI = args.ex.gu.I / kBlock, S = args.ex.gu.S, E = args.E;
     if (dense) {
-      units[0] = (S + E) * nbI;
+      units[0] = per * (S + E) * nbI;
       units[1] = (E + (S > 0 ? 1 : 0)) * (args.H / kBlock) * args.ks;
     } else {
       const bool lists = load_count(my_signal_flag(ctl, kSigPermuted)) != 0;
-      units[0] = lists ? (SPLIT ? 2 : 1) * load_count(&args.po.meta[kMetaUnitsGU]) : 0;
+      units[0] = lists ? per * load_count(&args.po.meta[kMetaUnitsGU]) : 0;
       units[1] = lists ? load_count(&args.po.meta[kMetaUnitsDN]) : 0;
     }
   }
@@ -3895,6 +4061,18 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
       bool done = true;
       if constexpr (SPLIT) {
         done = gateup_work_split(a.gu, g, red, &flag, ring, claiming(ReadyWait{nullptr, 0, nullptr}, queue, &ticket));
+      } else if constexpr (SMALL) {
+        const int c = g / per / nbI;
+        const bool routed = dense && c >= a.gu.S;  // a routed expert of the dense schedule
+        auto state = [&] { return dense_state(ctl, a.gu.offsets, c - a.gu.S, &flags[0]); };
+        const int st = routed ? state() : 0;
+        const ReadyWait ready =
+            dense ? ReadyWait{my_signal_flag(ctl, kSigQuant), 1, &ctl[kCtlError], kWaitTicks, true, 2}
+                  : ReadyWait{nullptr, 0, nullptr};
+        if (st == 2)
+          done = skip_small_unit<A16>(a.gu, g, &flag);
+        else
+          done = gateup_small_work<A16>(a.gu, g, part_sums, &flag, ring, claiming(ready, queue, &ticket), st == 1, state);
       } else if constexpr (BATCH) {
         gateup_batch_work<A16>(a.gu, g, &red[0][0], rings, claiming(ReadyWait{nullptr, 0, nullptr}, queue, &ticket));
       } else if (dense) {
@@ -3914,7 +4092,7 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
       if (done) {
         publish_fence();
         __syncthreads();
-        const int dc = dense ? dense_dn_of_gu(g / nbI, a.gu.S) : a.dn_of_gu[(SPLIT ? g >> 1 : g) / nbI];
+        const int dc = dense ? dense_dn_of_gu(g / per / nbI, a.gu.S) : a.dn_of_gu[g / per / nbI];
         if (threadIdx.x == 0) atomicAdd(&a.ready[(size_t)dc * a.ready_stride], 1);
       }
     } else {
@@ -3922,7 +4100,8 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
       const int sh = a.dn.S > 0 ? 1 : 0;
       const int st = dense && c >= sh ? dense_state(ctl, a.gu.offsets, c - sh, &flags[0]) : 0;
       if (st != 2) {
-        const int need = dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI);
+        const int need = (SMALL && A16 ? per : 1) *
+                         (dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI));
         const ReadyWait ready = claiming(
             ReadyWait{&a.ready[(size_t)c * a.ready_stride], need, &ctl[kCtlError]}, queue, &ticket);
         if constexpr (BATCH)
@@ -4014,6 +4193,9 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
     if constexpr (BATCH)
       for (int e = i; e < args.E; e += 256)
         __hip_atomic_store(&args.ranks.counts[e], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (SMALL)
+      for (int c = i; c < args.n_pairs; c += 256)  // the dense schedule's block counters
+        __hip_atomic_store(&args.ex.gu.pairs[c], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int c = i; c < args.n_ready; c += 256)  // the dense schedule's readiness counters
       __hip_atomic_store(&args.ex.ready[(size_t)c * args.ex.ready_stride], 0, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
@@ -4022,13 +4204,18 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
 
 template <bool SPLIT, bool A16 = false>
 __global__ __launch_bounds__(256, 2) void k_layer(LayerArgs args) {
-  layer_body<SPLIT, A16, false>(args);
+  layer_body<SPLIT, A16, false, false>(args);
 }
 
 // One workgroup per CU (the batch ring).
 template <bool A16>
 __global__ __launch_bounds__(256, 1) void k_layer_batch(LayerArgs args) {
-  layer_body<false, A16, true>(args);
+  layer_body<false, A16, true, false>(args);
+}
+
+template <bool A16>
+__global__ __launch_bounds__(256, 2) void k_layer_small(LayerArgs args) {
+  layer_body<false, A16, false, true>(args);
 }
 
 // =======================================================================================
@@ -5230,13 +5417,16 @@ inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
   size_t xn, partial, xq, xs, counts, offsets, meta, perm, inv, gu, dn, dn_of_gu, ready, ready_l, pairs, hq_r, hs_r,
-      hq_s, hs_s, st_r, st_s, h16_r, h16_s, d_r, d_s, p_r, p_s, spare, ctl, eperm, ecounts, total;
+      hq_s, hs_s, st_r, st_s, h16_r, h16_s, d_r, d_s, p_r, p_s, spare, ctl, pairs_l, eperm, ecounts, total;
   size_t total_ordered;  // what the stream-ordered form needs
   int nsplit;
   int ks;  // K parts of each down unit
   int ready_stride;  // ints between two readiness counters
   int dense;         // dense_experts
   int rows_r;        // routed rows of h and d: T*K, or E*T in the dense schedule
+  int parts;         // small_parts_wanted, or 1 where only whole blocks fit the device scratch
+  bool split;        // split_gate_up
+  int n_pairs_l;     // the small form's block counters in the dense schedule
   int n_ready_l;     // the single launch's own readiness counters (dense schedule), zeroed per call
 };
 
@@ -5250,28 +5440,25 @@ size_t max_chunks(const megamoe_desc& d, int copies, int chunk = kChunkRows) {
 
 // K parts of each down unit: when the routing can yield fewer than four down units per
 // workgroup of a reference grid (2 per CU on 256 CUs), the down GEMMs are split along K
-// into 2, 4 or 8 parts (dividing the K blocks), so the down phase keeps every workgroup
-// busy and its last units, which set the kernel's tail, are short.
+// into 2, 4 or 8 parts (dividing the K blocks) of at least kDownPartBlocks, so the down phase keeps
+// every workgroup busy and its last units, which set the kernel's tail, are short. Parts of few
+// K blocks (16 KB each) cost more in claims, readiness polls and partial rows than they spread. At
+// least 1 / 4 / 8 blocks: one and two tokens of DeepSeek-V3's shape 122 / 108 / 106 and 148 / 149 /
+// 139 us, of Qwen3-30B-A3B's 47 / 43 / 42 and 57 / 51 / 52, of GLM-5.3-Flash's 91 / 81 / 81 and 109 /
+// 108 / 105; four of Tiny's 28 / 24 / 24; 16 at least cost Mixtral's at 1 / 2 / 4 tokens 97 -> 105,
+// 143 -> 148, 200 -> 216.
 // Depends on the geometry only, so the numerics do not depend on the device.
+constexpr size_t kDownPartBlocks = 8;
 int down_splits(const megamoe_desc& d) {
   const size_t nbH = d.hidden / kBlock, nkb = d.intermediate / kBlock;
   const size_t hit = (size_t)(d.experts < (int64_t)d.tokens * d.topk ? d.experts : (int64_t)d.tokens * d.topk);
   const size_t units = (hit + (d.shared_experts > 0 ? 1 : 0)) * nbH;
   const size_t target = 4 * 512;
   int ks = 1;
-  while (ks < 8 && units * ks < target && nkb % (2 * ks) == 0) ks *= 2;
+  while (ks < 8 && units * ks < target && nkb % (2 * ks) == 0 && nkb / (2 * ks) >= kDownPartBlocks) ks *= 2;
   return ks;
 }
 
-// Whether the expert kernel works gate and up of each 128-row block as separate units
-// (k_experts<true>). Worth it only when the whole-block units cannot fill one round of a
-// reference grid (2 per CU on 256 CUs) even if every expert is hit, and the rows are long
-// enough (32 or more K blocks) for the hand-over between the halves to be cheap next to the
-// stream. A Mixtral-shaped layer (8 experts of 112 blocks: 896 units, 1.75 rounds) streams
-// its gate/up phase at 6.3-6.6 TB/s split and at 6.9-7.0 whole (per-unit timelines;
-// 231 -> 224 us for the stream-ordered expert kernel, 286 -> 282 us for the single launch),
-// and DeepSeek-V3, Kimi-K2 and Qwen3-30B-A3B measured 3-7% slower split. Depends on the
-// geometry only; both forms give the same bits.
 // Whether the expert units follow the dense schedule: every expert's gate/up and down units
 // over all T tokens, in lists known from the geometry, so they start as soon as x is
 // quantized instead of after the router, the routing and the permute (the single launch's
@@ -5289,8 +5476,39 @@ bool dense_experts(const megamoe_desc& d) {
   return d.tokens <= 16 && (int64_t)d.tokens * d.topk >= d.experts;
 }
 
-bool split_gate_up(const megamoe_desc& d) {
-  if (dense_experts(d)) return false;  // the dense schedule's units are whole blocks
+// Units per 128-row block of gate and up at T <= 16 (the small form, gateup_small_work; 1: whole
+// blocks): as many as make 1024 units, four per CU, of a call that hits as many experts as it can;
+// 512 once a unit is under 256 KB (each costs ~2 us of claims and hand-over beside its stream), and
+// up to 2048 while a unit keeps 512 KB (the routing leaves fewer blocks than the bound). The dense
+// schedule's blocks of under 512 KB stay whole: their time is the hand-overs' already. One call,
+// whole -> parts: DeepSeek-V3's shape at 1 / 2 / 4 / 8 tokens 125 -> 108, 156 -> 148, 215 -> 203, 338
+// -> 319 us; GLM-5.3-Flash's 89 -> 81, 114 -> 107, 159 -> 156, 229 -> 217; Mixtral's at 1 / 2 / 4 109
+// -> 97, 159 -> 142, 223 -> 200 (finer units also waste less on experts the routing turns out not to
+// pick); Qwen3-30B-A3B's at 1 / 4 / 16 47 -> 42, 63 -> 62, 112 -> 109. Depends on the geometry only.
+int small_parts_wanted(const megamoe_desc& d) {
+  const size_t entries = (size_t)d.tokens * d.topk, E = d.experts, nkb = d.hidden / kBlock;
+  const size_t blocks = ((entries < E ? entries : E) + d.shared_experts) * (size_t)(d.intermediate / kBlock);
+  const size_t bytes = (size_t)2 * kBlock * d.hidden;  // of a block of gate and up
+  if (d.tokens > 16 || (dense_experts(d) && bytes < (512u << 10))) return 1;
+  int p = 1;
+  while (p < 8 && nkb % p == 0 &&
+         (blocks * p < (bytes / p >= (256u << 10) ? 1024u : 512u) ||
+          (blocks * p < 2048 && bytes / (2 * p) >= (512u << 10))))
+    p *= 2;
+  return p;
+}
+
+// Whether the expert kernel works gate and up of each 128-row block as separate units
+// (k_experts<true>). Worth it only when the whole-block units cannot fill one round of a
+// reference grid (2 per CU on 256 CUs) even if every expert is hit, and the rows are long
+// enough (32 or more K blocks) for the hand-over between the halves to be cheap next to the
+// stream. A Mixtral-shaped layer (8 experts of 112 blocks: 896 units, 1.75 rounds) streams
+// its gate/up phase at 6.3-6.6 TB/s split and at 6.9-7.0 whole (per-unit timelines;
+// 231 -> 224 us for the stream-ordered expert kernel, 286 -> 282 us for the single launch),
+// and DeepSeek-V3, Kimi-K2 and Qwen3-30B-A3B measured 3-7% slower split. Depends on the
+// geometry only; both forms give the same bits.
+bool split_gate_up(const megamoe_desc& d, int parts) {
+  if (dense_experts(d) || parts > 1) return false;  // their units are blocks of both
   const size_t hit = (size_t)(d.experts < (int64_t)d.tokens * d.topk ? d.experts : (int64_t)d.tokens * d.topk);
   const size_t units = (hit + (size_t)d.shared_experts) * (size_t)(d.intermediate / kBlock);
   return units < 512 && d.hidden / kBlock >= 32;
@@ -5317,7 +5535,7 @@ bool batch_units(const megamoe_desc& d) {
          (d.tokens >= 208 || entries >= 16 * E || (large && d.tokens >= 128 && entries >= 4 * E));
 }
 
-Layout make_layout(const megamoe_desc& d) {
+Layout layout_with(const megamoe_desc& d, int parts) {
   Layout L{};
   const size_t T = d.tokens, H = d.hidden, E = d.experts, K = d.topk, I = d.intermediate, S = d.shared_experts;
   const bool batch = batch_units(d);
@@ -5371,9 +5589,12 @@ Layout make_layout(const megamoe_desc& d) {
     L.h16_r = base;
     L.h16_s = base + align_up(R * I * 2);
   }
-  const bool split = split_gate_up(d);  // staging of the separate gate and up units
-  L.st_r = take(split ? 2 * T * K * I * 2 : 0);
-  L.st_s = take(split ? 2 * T * S * I * 2 : 0);
+  // Staging: gate and up of the separate gate and up units, or h of the small form's.
+  const bool small = parts > 1;
+  L.parts = parts;
+  L.split = split_gate_up(d, parts);
+  L.st_r = take(L.split ? 2 * T * K * I * 2 : (small ? R * I * 2 : 0));
+  L.st_s = take(L.split ? 2 * T * S * I * 2 : (small ? T * S * I * 2 : 0));
   L.d_r = take(R * H * 2);
   L.d_s = take(T * H * 2);
   L.ks = down_splits(d);
@@ -5382,6 +5603,8 @@ Layout make_layout(const megamoe_desc& d) {
   L.spare = take(16 * (H > I * (S > 1 ? S : 1) ? H : I * (S > 1 ? S : 1)));
   L.ctl = take(kCtlInts * sizeof(int));  // the single-launch kernel's control words
   L.total_ordered = at;
+  L.n_pairs_l = small && L.dense ? (int)((E + S) * (I / kBlock)) : 0;
+  L.pairs_l = take((size_t)L.n_pairs_l * sizeof(int));  // the single launch's own, zeroed by each call
   // The batch form's permutation (TokenRanks): entries by expert behind the fewer partials that its
   // router leaves, where they fit; the experts' counts among the words that each call leaves zero.
   const size_t partials = align_up((size_t)L.nsplit * T * E * sizeof(double)), entries = batch ? E * T * sizeof(int) : 0;
@@ -5389,6 +5612,14 @@ Layout make_layout(const megamoe_desc& d) {
   L.ecounts = take(batch ? E * sizeof(int) : 0);
   L.total = at;
   return L;
+}
+
+// The small form's staging does not cost a layer its place in the fixed device scratch.
+Layout make_layout(const megamoe_desc& d) {
+  const Layout L = layout_with(d, small_parts_wanted(d));
+  if (L.parts == 1 || L.total_ordered <= (size_t)MEGAMOE_SCRATCH_BYTES) return L;
+  const Layout whole = layout_with(d, 1);
+  return whole.total_ordered <= (size_t)MEGAMOE_SCRATCH_BYTES ? whole : L;
 }
 
 int validate(const megamoe_desc* d) {
@@ -5542,6 +5773,7 @@ PermuteOut make_permute_out(const Layout& L, char* ws) {
                 (int*)(ws + L.ready),  (int*)(ws + L.pairs), L.ready_stride};
   // The dense schedule counts every expert's down chunk, hit or not (n_ready_l of them).
   po.ready_min = L.n_ready_l;
+  po.pairs_min = L.n_pairs_l;
   return po;
 }
 
@@ -5566,6 +5798,7 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   ga.swiglu = epi ? epi->swiglu : 0;
   ga.limit = epi ? epi->swiglu_limit : 0.0f;
   ga.dense = L.dense;
+  ga.parts = L.parts;
   ga.x16 = nullptr;  // set by the W8A16 form
   ga.h16_r = (uint16_t*)(ws + L.h16_r);
   ga.h16_s = (uint16_t*)(ws + L.h16_s);
@@ -5589,11 +5822,12 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   ea.ready_stride = po.ready_stride;
 }
 
-// The most gate/up and down units one call's lists can hold (the dense schedule's exactly).
-size_t expert_units_max(const megamoe_desc& d, const Layout& L, bool split, int chunk = kChunkRows) {
+// The most gate/up (`per` a 128-row block) and down units one call's lists can hold (the dense
+// schedule's exactly).
+size_t expert_units_max(const megamoe_desc& d, const Layout& L, int per, int chunk = kChunkRows) {
   const size_t nbI = d.intermediate / kBlock, nbH = d.hidden / kBlock, S = d.shared_experts, E = d.experts;
-  if (L.dense) return (S + E) * nbI + (E + (S > 0 ? 1 : 0)) * nbH * L.ks;
-  return (split ? 2 : 1) * max_chunks(d, (int)S, chunk) * nbI + max_chunks(d, S > 0 ? 1 : 0, chunk) * nbH * L.ks;
+  if (L.dense) return per * (S + E) * nbI + (E + (S > 0 ? 1 : 0)) * nbH * L.ks;
+  return per * max_chunks(d, (int)S, chunk) * nbI + max_chunks(d, S > 0 ? 1 : 0, chunk) * nbH * L.ks;
 }
 
 // The layer; with `blk`, the block form: RMSNorm of x before the router (the layer then
@@ -5655,11 +5889,16 @@ int forward_impl(const megamoe_desc* desc, const megamoe_tensors* t, hipStream_t
   const DownArgs& da = ea.dn;
   // As many workgroups as fit on the device at once, and no more than the most units the
   // routing can produce.
-  const bool split = !a16 && split_gate_up(d);
-  const size_t units_max = expert_units_max(d, L, split, chunk);
+  const bool split = !a16 && L.split;
+  const int parts = L.parts;
+  const size_t units_max = expert_units_max(d, L, split ? 2 : parts, chunk);
   const size_t resident = (size_t)di.cus * di.experts_per_cu;
   const unsigned grid = (unsigned)(units_max < resident ? units_max : resident);
-  if (a16)
+  if (parts > 1 && a16)
+    hipLaunchKernelGGL(k_experts_small<true>, dim3(grid), dim3(256), 0, st, ea);
+  else if (parts > 1)
+    hipLaunchKernelGGL(k_experts_small<false>, dim3(grid), dim3(256), 0, st, ea);
+  else if (a16)
     hipLaunchKernelGGL((k_experts<false, true>), dim3(grid), dim3(256), 0, st, ea);
   else if (split)
     hipLaunchKernelGGL(k_experts<true>, dim3(grid), dim3(256), 0, st, ea);
@@ -5748,10 +5987,11 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
 
   // As many workgroups as fit on the device at once, and no more than the most units the
   // queue can hold.
-  const bool split = !a16 && split_gate_up(d);
+  const bool split = !a16 && L.split;
   const bool batch = !split && batch_units(d);
+  const int parts = L.parts;
   const size_t units_max = (size_t)la.n_norm + la.n_router + T +
-                           expert_units_max(d, L, split, a16 ? kChunkRowsA16 : kChunkRows) +
+                           expert_units_max(d, L, split ? 2 : parts, a16 ? kChunkRowsA16 : kChunkRows) +
                            ((size_t)T * H + kCombineUnit - 1) / kCombineUnit;
   if (batch) {
     la.ranks = TokenRanks{(int*)(ws + L.ecounts), (int*)(ws + L.eperm), la.po.inv, T};
@@ -5760,6 +6000,8 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   la.dense = L.dense;
   la.n_ready = L.n_ready_l;
   if (L.dense) la.ex.ready = (int*)(ws + L.ready_l);
+  if (L.n_pairs_l) la.ex.gu.pairs = (int*)(ws + L.pairs_l);
+  la.n_pairs = L.n_pairs_l;
   const size_t resident = (size_t)di.cus * (batch ? 1 : di.layer_per_cu);
   const unsigned grid = (unsigned)(units_max < resident ? units_max : resident);
   // Router units taken by workgroup index: the first round of them, when there are 64 or more
@@ -5770,7 +6012,11 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   const char* rescue = getenv("MEGAMOE_FORCE_RESCUE");
   la.force_rescue = rescue && rescue[0] == '1' ? 1 : 0;
   if (mark(0) != hipSuccess) return MEGAMOE_ERR_HIP;
-  if (a16 && batch)
+  if (parts > 1 && a16)
+    hipLaunchKernelGGL(k_layer_small<true>, dim3(grid), dim3(256), 0, st, la);
+  else if (parts > 1)
+    hipLaunchKernelGGL(k_layer_small<false>, dim3(grid), dim3(256), 0, st, la);
+  else if (a16 && batch)
     hipLaunchKernelGGL(k_layer_batch<true>, dim3(grid), dim3(256), 0, st, la);
   else if (batch)
     hipLaunchKernelGGL(k_layer_batch<false>, dim3(grid), dim3(256), 0, st, la);
