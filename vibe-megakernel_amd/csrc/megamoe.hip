@@ -2151,6 +2151,11 @@ __device__ __forceinline__ void lds_wait(i32x4& a, i32x4& b) {
   asm volatile("s_waitcnt lgkmcnt(%c2)" : "+v"(a), "+v"(b) : "i"(N));
 }
 __device__ __forceinline__ void lds_arrived(i32x4& a, i32x4& b) { asm volatile("" : "+v"(a), "+v"(b)); }
+template <int OFF>
+__device__ __forceinline__ void lds_read_u2(uint2& v, uint32_t p) {
+  asm volatile("ds_read_b64 %0, %1 offset:%c2" : "=&v"(v) : "v"(p), "i"(OFF) : "memory");
+}
+__device__ __forceinline__ void lds_arrived(uint2& a) { asm volatile("" : "+v"(a)); }
 __device__ __forceinline__ void lds_arrived(float& a) { asm volatile("" : "+v"(a)); }
 
 // The weights of K block kb into a slot; past the last one (not live) as many loads from the spare
@@ -4468,9 +4473,9 @@ struct GateUpMxArgs {
 //   gate, up = bf16(l1); gate = min(gate, limit); up = clamp(up, +-limit)
 //   a = gate / (1 + exp(-gate)) * up * w_slot (fp32, megamoe.py:116-122)
 //   h = E4M3(a * 2^(127-e)), e = E8M0 exponent of the block's amax (megamoe.py:125-128)
-template <int NCT>
-__device__ void gateup_mx_epilogue(const GateUpMxArgs& a, int jb, const ChunkRows& cr, const f32x4 (&acc)[4][NCT],
-                                   uint8_t (*red8)[64]);
+template <int NCT, int RW>
+__device__ __forceinline__ void gateup_mx_epilogue(const GateUpMxArgs& a, int jb, const ChunkRows& cr,
+                                                   const f32x4 (&acc)[4][NCT], uint8_t (*red8)[RW]);
 
 template <int NCT, bool PAIR>
 __device__ void gateup_mx_unit(const GateUpMxArgs& a, int e, int jb, const ChunkRows& cr, int rot, uint8_t (*red8)[64],
@@ -4497,16 +4502,16 @@ __device__ void gateup_mx_unit(const GateUpMxArgs& a, int e, int jb, const Chunk
   }
   f32x4 acc[4][NCT];
   stream_gemm_mx<4, NCT, 2, PAIR>(op, H / kMxStageK, rot, ring, acc);
-  gateup_mx_epilogue<NCT>(a, jb, cr, acc, red8);
+  gateup_mx_epilogue(a, jb, cr, acc, red8);
 }
 
 // The epilogue of a 128-channel gate/up unit whose wave w holds gate and up channels
 // [32w, 32w + 32) of block jb for column tiles 0 .. NCT-1: SwiGLU, the E8M0 scale of each
 // row's 32 channels (within the wavefront), E4M3 h, and the four waves' scale bytes of a
 // row gathered into one dword.
-template <int NCT>
-__device__ void gateup_mx_epilogue(const GateUpMxArgs& a, int jb, const ChunkRows& cr, const f32x4 (&acc)[4][NCT],
-                                   uint8_t (*red8)[64]) {
+template <int NCT, int RW>
+__device__ __forceinline__ void gateup_mx_epilogue(const GateUpMxArgs& a, int jb, const ChunkRows& cr,
+                                                   const f32x4 (&acc)[4][NCT], uint8_t (*red8)[RW]) {
   const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15;
   const float L = a.limit;
@@ -4866,17 +4871,21 @@ __device__ void down_mx_work(const DownMxArgs& a, int v, int nwide, int* ready_c
 // Batch mode of the MXFP4 experts (tens of rows per expert, e.g. a rank's share under
 // expert parallelism): one workgroup per CU, every operand through LDS DMA.
 //   * weights: wave w streams its own 4 tiles (gate/up: 32 gate + 32 up rows of a
-//     128-channel block; down: 64 rows of a 256-row block) into a private ring of
-//     kBatchSlots stages, and their E8M0 scale rows (4-byte DMA) beside them;
-//   * activations: the chunk's (up to) 64 rows in 4 tiles of 16, tile w requested by wave w
-//     into a slot shared by the workgroup, with their E8M0 scale rows; each wave multiplies
-//     its weight tiles by all four tiles (64 MFMA accumulators);
+//     128-channel block; down: 64 rows of a 256-row block) into a private ring of stages,
+//     and their E8M0 scale rows beside them;
+//   * activations: the chunk's rows (up to 128) in tiles of 16, a quarter of them requested by
+//     each wave into slots shared by the workgroup, with their E8M0 scale rows; each wave
+//     multiplies its weight tiles by all of them;
 //   * one barrier per stage: after it every tile of the stage is in LDS and every wave has
-//     read the previous stage's slots, which the stage kBatchSlots - 1 ahead then refills.
+//     read the previous stage's slots.
 // No register load is in flight across the loop, so the compiler's wait counting cannot
 // force a drain; the LDS reads are inline asm, ordered by their own lgkmcnt wait. The K
 // rotation and the MFMA sequence of every output are the decode units', so a row's result
 // does not depend on the mode either.
+//
+// What bounds it is what a CU can take in (~29 KB/us). An expert's weights pass once per 128 rows and a
+// chunk brings only as many activation rows as it has (to 32): 3072 rows on 48 experts of H 7168, I 3072
+// take 433 us (chunks of 64 rows, all 64 brought: 491), 1152 rows 344 (369).
 // ---------------------------------------------------------------------------------------
 
 constexpr int kBatchSlots = 3;
@@ -4884,8 +4893,7 @@ constexpr int kBatchA = 4 * kTileBytes;      // a wave's four weight tiles of on
 constexpr int kBatchAs = 1024;               // their scale rows for a stage pair: 64 rows x 16 bytes
 constexpr int kBatchB = 4 * 2 * kTileBytes;  // four 16-row activation tiles x 256 bytes (16 KB)
 constexpr int kBatchBs = 1024;               // their scale rows for a stage pair: 64 rows x 16 bytes
-constexpr int kBatchRows = 64;               // rows per chunk
-constexpr int kBatchMinRows = 24;            // average rows per expert from which batch mode runs
+constexpr int kBatchRows = 128;              // rows per chunk
 
 struct BatchLds {
   uint8_t a[4][kBatchSlots][kBatchA];
@@ -4894,14 +4902,35 @@ struct BatchLds {
   uint8_t bs[kBatchSlots][kBatchBs];
 };
 
-// The per-lane addresses of one wave's loads, at stage 0 of the unit's K range.
+// The same LDS for chunks of 65-128 rows: two slots of each.
+struct BatchLds2 {
+  uint8_t a[4][2][kBatchA];
+  uint8_t as[4][2][kBatchAs];
+  uint8_t b[2][2 * kBatchB];
+  uint8_t bs[2][2 * kBatchBs];
+};
+static_assert(sizeof(BatchLds2) <= sizeof(BatchLds), "one LDS for both");
+
+// The per-lane addresses of one wave's loads, at stage 0 of the unit's K range, for a chunk of
+// NCT column tiles: wave w moves the activation rows 4*NCT*w .. +4*NCT-1.
+template <int NCT>
 struct BatchOps {
   OperandsMx<4, 1> w;        // weight tiles (a[], lda, spare); sa/b/sb unused
   const uint8_t* as;         // scale row of tile lane/16, row lane%16 (16 bytes: a stage pair)
-  const uint8_t* b[2];       // activation rows 8i + lane/8 of this wave's tile, at its swizzled chunk
-  const uint8_t* bs;         // lanes 0-15: scale row of this wave's tile row lane (a stage pair)
-  int bstage;                // activation bytes per stage (256)
+  const uint8_t* b[NCT / 2]; // activation rows 4*NCT*w + 8i + lane/8, at this lane's swizzled chunk
+  const uint8_t* bs;         // lanes below 4*NCT: scale row of this wave's row lane (a stage pair)
 };
+
+// The activation addresses: row r of the chunk is row(r) of x (ld bytes a row) and xs (sld).
+template <int NCT, class F>
+__device__ __forceinline__ void batch_mx_rows(BatchOps<NCT>& o, const uint8_t* x, size_t ld, const uint8_t* xs, size_t sld,
+                                              int n, F&& row) {
+  const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int i = 0; i < NCT / 2; ++i)
+    o.b[i] = x + (size_t)row(min(4 * NCT * w + 8 * i + (lane >> 3), n - 1)) * ld + (((lane & 7) ^ (lane >> 3)) << 4);
+  o.bs = xs + (size_t)row(min(4 * NCT * w + (lane & (NCT <= 4 ? 15 : 31)), n - 1)) * sld;
+}
 
 // One LDS DMA instruction: SIZE bytes per lane from src into dst + lane * SIZE (cached).
 template <int SIZE>
@@ -4918,23 +4947,27 @@ __device__ __forceinline__ void lds_dma(const uint8_t* src, uint8_t* dst) {
 // The weight tiles of stage pp (8 DMA instructions) into weight slot s; with `scales`, also
 // the E8M0 rows of the stage pair starting at the even stage pq (one 16-byte DMA: lane l
 // fetches row l % 16 of tile l / 16) into scale slot ss.
-__device__ __forceinline__ void batch_issue_w(BatchLds& L, const BatchOps& o, const LaneTile& lt, int w, int s, int pp,
+template <class LDS, int NCT>
+__device__ __forceinline__ void batch_issue_w(LDS& L, const BatchOps<NCT>& o, const LaneTile& lt, int w, int s, int pp,
                                               bool live, bool scales, int ss, int pq) {
   issue_a_mx<kNonTemporal>(L.a[w][s], o.w, lt, pp, live);
   if (scales) lds_dma<16>(o.as + 8 * pq, L.as[w][ss]);
 }
 
-// This wave's activation tile of stage pp (4 DMA instructions) into activation slot s;
-// with `scales`, also its tile's E8M0 rows for the stage pair at pq (lanes 0-15 only, each
-// 16 bytes) into scale slot ss.
-__device__ __forceinline__ void batch_issue_x(BatchLds& L, const BatchOps& o, int w, int s, int pp, bool scales, int ss,
+// This wave's activation rows of stage pp (NCT DMA instructions: 8 rows by 128 bytes each) into
+// activation slot s; with `scales`, also their E8M0 rows for the stage pair at pq (16 bytes a
+// row) into scale slot ss. A 16-row tile is 4 KB, its 128-byte halves 2 KB apart.
+template <class LDS, int NCT>
+__device__ __forceinline__ void batch_issue_x(LDS& L, const BatchOps<NCT>& o, int w, int s, int pp, bool scales, int ss,
                                               int pq) {
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      lds_dma<16>(o.b[q] + (size_t)pp * o.bstage + 128 * h, L.b[s] + w * 2 * kTileBytes + h * kTileBytes + q * 1024);
-  if (scales && opaque_lane() < 16) lds_dma<16>(o.bs + 8 * pq, L.bs[ss] + 256 * w);
+    for (int i = 0; i < NCT / 2; ++i) {
+      const int q = w * (NCT / 2) + i;  // group of 8 rows
+      lds_dma<16>(o.b[i] + (size_t)pp * kMxStageK + 128 * h, L.b[s] + (q >> 1) * 2 * kTileBytes + h * kTileBytes + (q & 1) * 1024);
+    }
+  if (scales && opaque_lane() < 4 * NCT) lds_dma<16>(o.bs + 8 * pq, L.bs[ss] + 64 * NCT * w);
 }
 
 // Weights run three stages ahead and activations two, in rings of three slots; the E8M0
@@ -4944,13 +4977,14 @@ __device__ __forceinline__ void batch_issue_x(BatchLds& L, const BatchOps& o, in
 // and every wave has read the activation slot of stage p - 1); request activations p + 2
 // into that slot; read stage p; request weights p + 3 into the weight slot just read; the
 // MFMAs. The loads go out in the order x(p+2), w(p+3) and those issued after x(p) are w(p+1),
-// x(p+1), w(p+2): 21 instructions for even p and 22 for odd p (a pair's scales ride with its
-// even stage), 4 and 13 at p = 0 and 1 after the prologue's w0 w1 w2 x0 x1. Waiting for x(p)
+// x(p+1), w(p+2): 17 + NCT instructions for even p and 18 + NCT for odd p (a pair's scales ride
+// with its even stage), NCT and 9 + NCT at p = 0 and 1 after the prologue's w0 w1 w2 x0 x1. Waiting for x(p)
 // also completes w(p) and both scale pairs of stage p, issued before it. The unroll of six
 // keeps every slot index a compile-time constant. The stage count and the rotation are even
 // (the host runs batch mode only then), so a pair never wraps.
-__device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps& o, int nst, int rot,
-                                                     f32x4 (&acc)[4][4],
+template <int NCT>
+__device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps<NCT>& o, int nst, int rot,
+                                                     f32x4 (&acc)[4][NCT],
                                                      const ReadyWait& ready = ReadyWait{nullptr, 0, nullptr}) {
   constexpr int S = kBatchSlots, U = 6;
   static_assert(S == 3, "three-slot rings: weights three stages ahead, activations two");
@@ -4968,7 +5002,7 @@ __device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NCT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Weights (and their scales) first: they do not depend on the readiness wait.
 #pragma unroll
   for (int i = 0; i < 3; ++i)
@@ -4989,19 +5023,19 @@ __device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps
       const int p = p0 + s;
       if (p >= 2) {
         if constexpr (s % 2 == 0)
-          wait_vmem<21>();
+          wait_vmem<17 + NCT>();
         else
-          wait_vmem<22>();
+          wait_vmem<18 + NCT>();
       } else if (p == 1) {
-        wait_vmem<13>();
+        wait_vmem<9 + NCT>();
       } else {
-        wait_vmem<4>();
+        wait_vmem<NCT>();
       }
       __builtin_amdgcn_s_barrier();
       batch_issue_x(L, o, w, (s + 2) % S, phys(min(p + 2, nst - 1)), s % 2 == 0, ((s + 2) / 2) % S, pair_of(p + 2));
       i32x4 lo[4], hi[4];
-      uint2 saw[4], sbw[4];
-      StageMx<4, 4> st;
+      uint2 saw[4], sbw[NCT];
+      StageMx<4, NCT> st;
       if (p < nst) {
         read_slot_mx<4>(lo, hi, a_lds + (s % S) * kBatchA + lt.rd0, a_lds + (s % S) * kBatchA + lt.rd1);
         const uint32_t half = 8 * (s % 2);
@@ -5012,7 +5046,7 @@ __device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps
         for (int t = 0; t < 4; ++t)
           asm volatile("ds_read_b64 %0, %1" : "=v"(saw[t]) : "v"(asb + 256 * t) : "memory");
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NCT; ++c) {
           asm volatile("ds_read_b64 %0, %1" : "=v"(sbw[c]) : "v"(bsb + 256 * c) : "memory");
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
@@ -5025,11 +5059,9 @@ __device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps
             st.b[c][h] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
           }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(saw[0]), "+v"(saw[1]), "+v"(saw[2]), "+v"(saw[3]), "+v"(sbw[0]), "+v"(sbw[1]),
-                       "+v"(sbw[2]), "+v"(sbw[3]));
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(saw[0]), "+v"(saw[1]), "+v"(saw[2]), "+v"(saw[3]));
 #pragma unroll
-        for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(st.b[c][0]), "+v"(st.b[c][1]));
+        for (int c = 0; c < NCT; ++c) asm volatile("" : "+v"(sbw[c]), "+v"(st.b[c][0]), "+v"(st.b[c][1]));
       }
       // The weight slot of stage p is read (its lgkmcnt wait is above): refill it.
       batch_issue_w(L, o, lt, w, s % S, phys(min(p + 3, nst - 1)), p + 3 < nst, (s + 3) % 2 == 0, ((s + 3) / 2) % S,
@@ -5037,16 +5069,129 @@ __device__ __forceinline__ void stream_gemm_mx_batch(BatchLds& L, const BatchOps
       if (p < nst) mfma_stage_mx(lo, hi, st, saw, sbw, shift, acc);
     });
   }
+  wait_vmem<0>();  // the tail's loads: the next unit may lay the LDS out for more rows
 }
 
-// Batch gate/up unit: 128-channel block jb of gate and up for the chunk's rows (at most 64):
+// The stream of chunks of 65-128 rows (NCT 6 or 8): two slots of each operand fill the LDS. A
+// stage's weights are requested two stages ahead, into the wave's own slot as soon as it has read
+// it, its activations one, after the barrier that ends the last reads of their slot. Order: w0 w1
+// x0, then at stage p x(p+1), w(p+2): only w(p+1) was issued after x(p) when stage p is waited
+// for, 8 instructions (9 with the scales of an even stage p+1). The activation tiles are read from
+// LDS two at a time, the next two's reads under the MFMAs (the registers hold 32 accumulators a
+// row tile).
+template <int NCT>
+__device__ __forceinline__ void stream_gemm_mx_batch2(BatchLds2& L, const BatchOps<NCT>& o, int nst, int rot,
+                                                      f32x4 (&acc)[4][NCT], const ReadyWait& ready) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = opaque_lane(), r = lane & 15;
+  auto phys = [nst, rot](int p) {
+    const int q = p + rot;
+    return q >= nst ? q - nst : q;
+  };
+  auto pair_of = [&](int q) { return phys(2 * min(q / 2, nst / 2 - 1)); };
+  const LaneTile lt = lane_tile(o.w.lda);
+  const int shift = 8 * (lane >> 4);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  batch_issue_w(L, o, lt, w, 0, phys(0), true, true, 0, pair_of(0));
+  batch_issue_w(L, o, lt, w, 1, phys(min(1, nst - 1)), 1 < nst, false, 0, 0);
+  wait_ready(ready);
+  batch_issue_x(L, o, w, 0, phys(0), true, 0, pair_of(0));
+  const uint32_t a_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&L.a[w][0][0];
+  const uint32_t as_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&L.as[w][0][0];
+  const uint32_t b_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&L.b[0][0];
+  const uint32_t bs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&L.bs[0][0];
+  const int rr = r & 7, g = lane >> 4;
+  const uint32_t brow = (uint32_t)((r >> 3) * 1024 + rr * kBlock);
+  for (int p0 = 0; p0 < nst; p0 += 4) {
+    static_for<0, 4>([&](auto si) {
+      constexpr int s = decltype(si)::value;
+      const int p = p0 + s;
+      if (p == 0)
+        wait_vmem<0>();
+      else if constexpr (s % 2 == 0)
+        wait_vmem<8>();
+      else
+        wait_vmem<9>();
+      __builtin_amdgcn_s_barrier();
+      batch_issue_x(L, o, w, (s + 1) % 2, phys(min(p + 1, nst - 1)), s % 2 == 1, ((s + 1) / 2) % 2, pair_of(p + 1));
+      i32x4 lo[4], hi[4];
+      uint2 saw[4], sbw[NCT];
+      i32x4 x[NCT][4];
+      const uint32_t half = 8 * (s % 2);
+      const uint32_t pb0 = b_lds + (s % 2) * 2 * kBatchB + brow + ((g ^ rr) << 4);
+      const uint32_t pb1 = b_lds + (s % 2) * 2 * kBatchB + brow + (((g + 4) ^ rr) << 4);
+      const uint32_t bsb = bs_lds + ((s / 2) % 2) * 2 * kBatchBs + 16 * r + half;
+      auto read_tile = [&](auto c) {
+        lds_read_u2<c.value * 256>(sbw[c.value], bsb);
+        lds_read2<c.value * 2 * kTileBytes>(x[c.value][0], x[c.value][1], pb0, pb1);
+        lds_read2<c.value * 2 * kTileBytes + kTileBytes>(x[c.value][2], x[c.value][3], pb0, pb1);
+      };
+      if (p < nst) {
+        const uint32_t asb = as_lds + ((s / 2) % 2) * kBatchAs + 16 * r + half;
+        static_for<0, 4>([&](auto q) { lds_read_u2<q.value * 256>(saw[q.value], asb); });
+        read_slot_mx<4>(lo, hi, a_lds + (s % 2) * kBatchA + lt.rd0, a_lds + (s % 2) * kBatchA + lt.rd1);
+        static_for<0, 4>([&](auto q) { lds_arrived(saw[q.value]); });
+      }
+      // The weight slot of stage p is read: refill it.
+      batch_issue_w(L, o, lt, w, s % 2, phys(min(p + 2, nst - 1)), p + 2 < nst, s % 2 == 0, ((s + 2) / 2) % 2,
+                    pair_of(p + 2));
+      if (p < nst) {
+        int sa0[4], sa1[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          sa0[q] = (int)((saw[q].x >> shift) & 0xffu);
+          sa1[q] = (int)((saw[q].y >> shift) & 0xffu);
+        }
+        static_for<0, 2>(read_tile);
+        static_for<0, NCT / 2>([&](auto ci) {
+          constexpr int c0 = 2 * decltype(ci)::value;
+          if constexpr (c0 + 2 < NCT) static_for<c0 + 2, c0 + 4>(read_tile);
+          // Ten reads (two tiles) stay pending, none before the last two.
+          lds_wait<(c0 + 2 < NCT ? 10 : 0)>(x[c0][0], x[c0][1]);
+#pragma unroll
+          for (int c = c0; c < c0 + 2; ++c) {
+            lds_arrived(sbw[c]);
+            lds_arrived(x[c][0], x[c][1]);
+            lds_arrived(x[c][2], x[c][3]);
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int c = c0; c < c0 + 2; ++c) {
+              const i32x8 bx = __builtin_shufflevector(x[c][2 * h], x[c][2 * h + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+              const int sb = (int)(((h ? sbw[c].y : sbw[c].x) >> shift) & 0xffu);
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                acc[q][c] = mfma_e2m1_e4m3(h ? hi[q] : lo[q], bx, acc[q][c], h ? sa1[q] : sa0[q], sb);
+            }
+        });
+      }
+    });
+  }
+  wait_vmem<0>();  // the tail's loads: the next unit may lay the LDS out for fewer rows
+}
+
+template <int NCT>
+__device__ __forceinline__ void batch_mx_gemm(BatchLds& L, const BatchOps<NCT>& o, int nst, int rot,
+                                              f32x4 (&acc)[4][NCT], const ReadyWait& ready) {
+  if constexpr (NCT <= 4)
+    stream_gemm_mx_batch<NCT>(L, o, nst, rot, acc, ready);
+  else
+    stream_gemm_mx_batch2<NCT>(*reinterpret_cast<BatchLds2*>(&L), o, nst, rot, acc, ready);
+}
+
+// Batch gate/up unit: 128-channel block jb of gate and up for the chunk's rows (at most 16*NCT):
 // wave w holds gate and up channels [32w, 32w + 32), as the decode unit.
-__device__ void gateup_mx_batch(const GateUpMxArgs& a, int e, int jb, const ChunkRows& cr, int rot, BatchLds& L,
-                                uint8_t (*red8)[64]) {
+template <int NCT>
+__device__ __forceinline__ void gateup_mx_batch(const GateUpMxArgs& a, int e, int jb, const ChunkRows& cr, int rot, BatchLds& L,
+                                uint8_t (*red8)[kBatchRows]) {
   const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int H = a.H, lda = H / 2, sld = H / 32;
   const size_t gate0 = (size_t)e * 2 * a.I + (size_t)jb * kBlock + 32 * w, up0 = gate0 + a.I;
-  BatchOps o;
+  BatchOps<NCT> o;
   o.w.lda = lda;
   o.w.spare = a.spare;
 #pragma unroll
@@ -5059,43 +5204,34 @@ __device__ void gateup_mx_batch(const GateUpMxArgs& a, int e, int jb, const Chun
     const size_t row = (t < 2 ? gate0 + 16 * t : up0 + 16 * (t - 2)) + (lane & 15);
     o.as = a.l1s + row * sld;
   }
-  const int chunk16 = ((lane & 7) ^ (lane >> 3)) << 4;
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-    o.b[q] = a.x + (size_t)row_token(cr, min(16 * w + 8 * q + (lane >> 3), cr.n - 1)) * H + chunk16;
-  o.bs = a.xs + (size_t)row_token(cr, min(16 * w + (lane & 15), cr.n - 1)) * sld;
-  o.bstage = kMxStageK;
-  f32x4 acc[4][4];
-  stream_gemm_mx_batch(L, o, H / kMxStageK, rot, acc);
-  gateup_mx_epilogue<4>(a, jb, cr, acc, red8);
+  batch_mx_rows(o, a.x, (size_t)H, a.xs, (size_t)sld, cr.n, [&cr](int r) { return row_token(cr, r); });
+  f32x4 acc[4][NCT];
+  batch_mx_gemm<NCT>(L, o, H / kMxStageK, rot, acc, ReadyWait{nullptr, 0, nullptr});
+  gateup_mx_epilogue(a, jb, cr, acc, red8);
 }
 
 // Batch down unit: down rows [256 j2, +256) over K part kp for the chunk's rows; wave w
 // holds rows 64w .. 64w+63 of the block.
-__device__ void down_mx_batch(const DownMxArgs& a, int e, int j2, int kp, const ChunkRows& cr, int rot,
+template <int NCT>
+__device__ __forceinline__ void down_mx_batch(const DownMxArgs& a, int e, int j2, int kp, const ChunkRows& cr, int rot,
                               const ReadyWait& ready, BatchLds& L) {
   const int lane = opaque_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15;
   const int I = a.I, lda = I / 2, sld = I / 32, nstp = I / kMxStageK / a.ks, p0 = kp * nstp;
   const size_t row0 = (size_t)e * a.H + (size_t)j2 * 256 + 64 * w;
-  BatchOps o;
+  BatchOps<NCT> o;
   o.w.lda = lda;
   o.w.spare = a.spare;
 #pragma unroll
   for (int t = 0; t < 4; ++t) o.w.a[t] = a.l2 + (row0 + 16 * t) * lda + (size_t)p0 * kBlock;
   o.as = a.l2s + (row0 + 16 * (lane >> 4) + (lane & 15)) * sld + 8 * p0;
-  const int chunk16 = ((lane & 7) ^ (lane >> 3)) << 4;
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-    o.b[q] = a.hq + (size_t)(cr.row0 + min(16 * w + 8 * q + (lane >> 3), cr.n - 1)) * I + (size_t)p0 * kMxStageK +
-             chunk16;
-  o.bs = a.hs + (size_t)(cr.row0 + min(16 * w + (lane & 15), cr.n - 1)) * a.hs_ld + 8 * p0;
-  o.bstage = kMxStageK;
-  f32x4 acc[4][4];
-  stream_gemm_mx_batch(L, o, nstp, rot, acc, ready);
+  batch_mx_rows(o, a.hq + (size_t)cr.row0 * I + (size_t)p0 * kMxStageK, (size_t)I,
+                a.hs + (size_t)cr.row0 * a.hs_ld + 8 * p0, (size_t)a.hs_ld, cr.n, [](int r) { return r; });
+  f32x4 acc[4][NCT];
+  batch_mx_gemm<NCT>(L, o, nstp, rot, acc, ready);
   float* pd = a.pd + (size_t)kp * a.T * a.K * a.H;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < NCT; ++c) {
     const int col = 16 * c + lr;
     if (col < cr.n) {
 #pragma unroll
@@ -5188,10 +5324,10 @@ __global__ __launch_bounds__(256, 2) void k_experts_mx(ExpertMxArgs args) {
 
 
 // The batch-mode expert kernel: the queue, claims and readiness waits of k_experts_mx, one
-// workgroup per CU, with the batch units (chunks of at most 64 rows; down units of 256 rows).
+// workgroup per CU, with the batch units (chunks of at most 128 rows; down units of 256 rows).
 __global__ __launch_bounds__(256, 1) void k_experts_mx_batch(ExpertMxArgs args) {
   typedef const __attribute__((address_space(4))) ExpertMxArgs* ArgsPtr;
-  __shared__ uint8_t red8[4][64];
+  __shared__ uint8_t red8[4][kBatchRows];
   __shared__ __attribute__((aligned(16))) BatchLds lds;
   __shared__ int slot, bnd[kXcds + 1];
   int* meta = args.gu.meta;
@@ -5224,7 +5360,15 @@ __global__ __launch_bounds__(256, 1) void k_experts_mx_batch(ExpertMxArgs args) 
       const int4 ch = a.gu.chunks[c];
       const ChunkRows cr{ch.z, ch.y, a.gu.perm, a.gu.K};
       const int nst = a.gu.H / kMxStageK;
-      gateup_mx_batch(a.gu, ch.x, jb, cr, mx_rotation((ch.x + a.gu.ebase) * nbI + jb, nst), lds, red8);
+      const int rot = mx_rotation((ch.x + a.gu.ebase) * nbI + jb, nst);
+      if (cr.n <= 32)
+        gateup_mx_batch<2>(a.gu, ch.x, jb, cr, rot, lds, red8);
+      else if (cr.n <= 64)
+        gateup_mx_batch<4>(a.gu, ch.x, jb, cr, rot, lds, red8);
+      else if (cr.n <= 96)
+        gateup_mx_batch<6>(a.gu, ch.x, jb, cr, rot, lds, red8);
+      else
+        gateup_mx_batch<8>(a.gu, ch.x, jb, cr, rot, lds, red8);
       publish_fence();
       __syncthreads();
       if (threadIdx.x == 0) atomicAdd(&a.ready[a.dn_of_gu[c]], 1);
@@ -5236,8 +5380,15 @@ __global__ __launch_bounds__(256, 1) void k_experts_mx_batch(ExpertMxArgs args) 
       const ChunkRows cr{ch.z, ch.y, a.dn.perm, a.dn.K};
       const ReadyWait ready{&a.ready[c], nbI, &meta[kMetaError]};
       const int nstp = a.dn.I / kMxStageK / ks;
-      down_mx_batch(a.dn, ch.x, j2, kp, cr, mx_rotation(((ch.x + a.dn.ebase) * nbH2 + j2) * ks + kp, nstp), ready,
-                    lds);
+      const int rot = mx_rotation(((ch.x + a.dn.ebase) * nbH2 + j2) * ks + kp, nstp);
+      if (cr.n <= 32)
+        down_mx_batch<2>(a.dn, ch.x, j2, kp, cr, rot, ready, lds);
+      else if (cr.n <= 64)
+        down_mx_batch<4>(a.dn, ch.x, j2, kp, cr, rot, ready, lds);
+      else if (cr.n <= 96)
+        down_mx_batch<6>(a.dn, ch.x, j2, kp, cr, rot, ready, lds);
+      else
+        down_mx_batch<8>(a.dn, ch.x, j2, kp, cr, rot, ready, lds);
     }
     if (threadIdx.x == 0) slot = next;
     __syncthreads();
@@ -6105,6 +6256,19 @@ LayoutMx make_layout_mx(const megamoe_desc& d) {
   return L;
 }
 
+// Whether the stream-ordered experts run as batch units (k_experts_mx_batch, one workgroup per CU) or
+// as decode units (two): from 24 rows an expert on average, and from 8 where the experts' weights are
+// large enough (8M per matrix and more) that the batch units' few long ones still balance. One call,
+// decode -> batch at 8 / 12 / 16 / 24 rows an expert: 48 experts of H 7168, I 3072 333 -> 322, 363 ->
+// 326, 383 -> 336, 369 -> 344 us (at 4: 299 -> 295); 96 of them 600 -> 600, 662 -> 626, 727 -> 634,
+// 703 -> 660 (at 4: 536 -> 572); 48 of 2048 by 2048 119 -> 129, 137 -> 132, 142 -> 136, 157 -> 146; 128
+// of 2048 by 1024 106 -> 132, 114 -> 135, 144 -> 159, 216 -> 201. Both give the same bits.
+bool batch_units_mx(const megamoe_desc& d, const LayoutMx& L) {
+  const bool large = (int64_t)d.hidden * d.intermediate >= ((int64_t)8 << 20);
+  return (int64_t)d.tokens * d.topk >= (int64_t)(large ? 8 : 24) * d.experts && (d.hidden / kMxStageK) % 2 == 0 &&
+         (d.intermediate / kMxStageK / L.ks) % 2 == 0;
+}
+
 // The MXFP4 expert kernels' arguments over workspace `ws`.
 void fill_expert_mx_args(const megamoe_desc& d, const LayoutMx& L, const megamoe_mx_tensors* t, char* ws,
                          const PermuteOut& po, float limit, int64_t base, bool direct, ExpertMxArgs& ea) {
@@ -6160,11 +6324,9 @@ int forward_mx_impl(const megamoe_desc* desc, float limit, const megamoe_mx_tens
   PermuteOut po{(int*)(ws + L.counts), (int*)(ws + L.offsets), (int*)(ws + L.meta), (int*)(ws + L.perm),
                 (int*)(ws + L.inv),    (int4*)(ws + L.gu),     (int4*)(ws + L.dn),  (int*)(ws + L.dn_of_gu),
                 (int*)(ws + L.ready)};
-  // Batch mode (k_experts_mx_batch) when the rows per expert average kBatchMinRows or more:
-  // chunks of up to 64 rows, down units of 256 rows, no wide units; the lists in expert
-  // order and the units claimed from per-XCD queues.
-  const bool batch = (int64_t)T * K >= (int64_t)kBatchMinRows * E && (H / kMxStageK) % 2 == 0 &&
-                     (I / kMxStageK / L.ks) % 2 == 0;
+  // Batch mode (k_experts_mx_batch): chunks of up to kBatchRows rows, down units of 256 rows, no wide
+  // units; the lists in expert order and the units claimed from per-XCD queues.
+  const bool batch = batch_units_mx(d, L);
   if (batch) po.xcd = (int*)(ws + L.xcd);
   if ((rc = launch_permute(t->topk_idx, base, T, K, E, 0, nbI, batch ? nbH / 2 : nbH, L.ks,
                            batch ? kBatchRows : kChunkRowsMx, batch ? 2 : 1, po, st)))
@@ -6223,8 +6385,7 @@ int forward_mx_layer_impl(const megamoe_desc* desc, float limit, const megamoe_m
   if (t->workspace_bytes < L.total) return MEGAMOE_ERR_WORKSPACE;
   const int T = d.tokens, H = d.hidden, E = d.experts, K = d.topk, I = d.intermediate;
   const int nbI = I / kBlock, nbH = H / kBlock;
-  const bool batch = (int64_t)T * K >= (int64_t)kBatchMinRows * E && (H / kMxStageK) % 2 == 0 &&
-                     (I / kMxStageK / L.ks) % 2 == 0;
+  const bool batch = batch_units_mx(d, L);
   const int tile_waves = permute_tile_waves(T, E, 256, kPermuteLdsInts);
   if (batch || tile_waves < 0) {  // the stream-ordered kernels, between the caller's two events
     if (mark(0) != hipSuccess) return MEGAMOE_ERR_HIP;
