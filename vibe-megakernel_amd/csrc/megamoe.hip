@@ -1907,8 +1907,9 @@ __device__ __forceinline__ void compute_stage(uint32_t slot, const LaneTile& lt,
 // first weights, which only makes the first stage's vmcnt wait below more conservative).
 //
 // The stream starts at K block `rot` and wraps around (any rot in [0, nkb); callers derive
-// it from the weight block, so a row's sum does not depend on the form of unit that takes it). Units that run at the same time then read different K blocks of
-// their weight rows: with every workgroup at the same K block, the addresses in flight
+// it from the unit's place, or from the weight block where units of two forms share a geometry,
+// so that a row's sum does not depend on the form that takes it). Units that run at the same time
+// then read different K blocks of their weight rows: with every workgroup at the same K block, the addresses in flight
 // differ only in their high bits (multiples of the row length, 4 KiB for some models), and
 // the HBM channels serve them unevenly (about 6% slower on a Mixtral-shaped layer). The
 // fp32 sum over K blocks then runs in a rotated order, the same on every call.
@@ -2394,7 +2395,8 @@ struct GateUpArgs {
   int swiglu;                   // 0: fp32 product rounded once; 1: bf16 silu, bf16 product
   float limit;                  // > 0: SwiGLU clamp (gate above, up both sides)
   int dense;                    // the dense schedule: units from dense_gu_chunk, h rows e*T + t
-  int parts;                    // the small form: units per 128-row block (2, 4 or 8)
+  int parts;                    // the small form: units per 128-row block (2, 4 or 8); 1: whole blocks; 0: whole, in a
+                                // geometry of the batch form
   const uint16_t* x16;          // W8A16: the bf16 rows [T, H] the experts read (x, or the normalized x)
   uint16_t* h16_r;              // W8A16: bf16 h of the routed rows [rows_r, I]
   uint16_t* h16_s;              // W8A16: of the shared rows [T, S*I]
@@ -2573,7 +2575,10 @@ __device__ __forceinline__ void gateup_work(const GateUpArgs& a, int u, float (*
   const int nbI = a.I / kBlock, nkb = a.H / kBlock;
   const int4 ch = a.dense ? dense_gu_chunk(u / nbI, a.E, a.S, a.T, nbI) : a.chunks[u / nbI];
   const int j = u % nbI, jb = ch.w + j;
-  const int rot = (ch.x * nbI + jb) % nkb;  // keyed by the weight block (see stream_gemm)
+  // Concurrent units start at different K blocks: by unit, or by weight block where the single
+  // launch works the geometry in batch units, which do so (by block there too, GLM-5.3-Flash's shape at
+  // 37 tokens takes 422.4 us instead of 420.8).
+  const int rot = (a.parts ? u : ch.x * nbI + jb) % nkb;
   const uint8_t *wg, *wu;
   const float *sg, *su;
   uint8_t* hq;
@@ -5949,7 +5954,7 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   ga.swiglu = epi ? epi->swiglu : 0;
   ga.limit = epi ? epi->swiglu_limit : 0.0f;
   ga.dense = L.dense;
-  ga.parts = L.parts;
+  ga.parts = L.parts == 1 && batch_units(d) ? 0 : L.parts;
   ga.x16 = nullptr;  // set by the W8A16 form
   ga.h16_r = (uint16_t*)(ws + L.h16_r);
   ga.h16_s = (uint16_t*)(ws + L.h16_s);
