@@ -169,6 +169,24 @@ def test_mx_one_call_is_one_kernel_launch():
     assert case.max_gpu_launches == 1
 
 
+@pytest.mark.parametrize("rows,kernel", [(8, "k_layer_mx"), (11, "k_layer_mx"), (12, "k_experts_mx_batch"),
+                                         (24, "k_experts_mx_batch")])
+def test_mx_single_launch_keeps_one_launch_below_its_line(rows, kernel):
+    """Large experts (8M weights a matrix): one launch below 12 rows an expert, the stream-ordered
+    batch units from there, with the bits of megamoe_mx_forward, whose own line lies lower."""
+    case = C.development(C.case(MXCASE), tokens=2 * rows, experts=4, topk=2, hidden=2048, intermediate=4096)
+    _log(f"mx single launch line rows={rows}")
+    values = workloads.make_inputs(case, 41, DEV)
+    one, three = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
+    one(values)  # the workspace is made (and zeroed) on the first call
+    y, kernels = _kernels_of(lambda: one(values)["y"])
+    want = three(values)["y"]
+    torch.cuda.synchronize()
+    assert any(kernel in k for k in kernels), kernels
+    assert len(kernels) == (1 if kernel == "k_layer_mx" else 3), kernels
+    assert torch.equal(y, want)
+
+
 def _bad_ids_cases():
     base = C.case(MXCASE)
     # The decode geometry runs k_layer_mx; the batch-shaped one (100 rows per expert, an even

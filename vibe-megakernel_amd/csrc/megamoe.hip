@@ -6268,9 +6268,15 @@ LayoutMx make_layout_mx(const megamoe_desc& d) {
 // 326, 383 -> 336, 369 -> 344 us (at 4: 299 -> 295); 96 of them 600 -> 600, 662 -> 626, 727 -> 634,
 // 703 -> 660 (at 4: 536 -> 572); 48 of 2048 by 2048 119 -> 129, 137 -> 132, 142 -> 136, 157 -> 146; 128
 // of 2048 by 1024 106 -> 132, 114 -> 135, 144 -> 159, 216 -> 201. Both give the same bits.
-bool batch_units_mx(const megamoe_desc& d, const LayoutMx& L) {
+//
+// `single`: for megamoe_mx_layer_forward, whose other form is one launch (k_layer_mx) that pays no
+// launch gaps: from 12 rows of large experts. k_layer_mx -> the three launches at 8 / 10 or 12 / 16 rows:
+// 48 experts of H 7168, I 3072 314 -> 322, 343 -> 325, 381 -> 329 us; 384 of them 2467 -> 2400, 2717 ->
+// 2470, 3010 -> 2575; 64 of H 4096, I 2048 187 -> 192, 200 -> 194, 220 -> 203.
+bool batch_units_mx(const megamoe_desc& d, const LayoutMx& L, bool single) {
   const bool large = (int64_t)d.hidden * d.intermediate >= ((int64_t)8 << 20);
-  return (int64_t)d.tokens * d.topk >= (int64_t)(large ? 8 : 24) * d.experts && (d.hidden / kMxStageK) % 2 == 0 &&
+  const int rows = !large ? 24 : (single ? 12 : 8);
+  return (int64_t)d.tokens * d.topk >= (int64_t)rows * d.experts && (d.hidden / kMxStageK) % 2 == 0 &&
          (d.intermediate / kMxStageK / L.ks) % 2 == 0;
 }
 
@@ -6331,7 +6337,7 @@ int forward_mx_impl(const megamoe_desc* desc, float limit, const megamoe_mx_tens
                 (int*)(ws + L.ready)};
   // Batch mode (k_experts_mx_batch): chunks of up to kBatchRows rows, down units of 256 rows, no wide
   // units; the lists in expert order and the units claimed from per-XCD queues.
-  const bool batch = batch_units_mx(d, L);
+  const bool batch = batch_units_mx(d, L, false);
   if (batch) po.xcd = (int*)(ws + L.xcd);
   if ((rc = launch_permute(t->topk_idx, base, T, K, E, 0, nbI, batch ? nbH / 2 : nbH, L.ks,
                            batch ? kBatchRows : kChunkRowsMx, batch ? 2 : 1, po, st)))
@@ -6390,7 +6396,7 @@ int forward_mx_layer_impl(const megamoe_desc* desc, float limit, const megamoe_m
   if (t->workspace_bytes < L.total) return MEGAMOE_ERR_WORKSPACE;
   const int T = d.tokens, H = d.hidden, E = d.experts, K = d.topk, I = d.intermediate;
   const int nbI = I / kBlock, nbH = H / kBlock;
-  const bool batch = batch_units_mx(d, L);
+  const bool batch = batch_units_mx(d, L, true);
   const int tile_waves = permute_tile_waves(T, E, 256, kPermuteLdsInts);
   if (batch || tile_waves < 0) {  // the stream-ordered kernels, between the caller's two events
     if (mark(0) != hipSuccess) return MEGAMOE_ERR_HIP;
