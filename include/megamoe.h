@@ -307,8 +307,8 @@ int megamoe_mx_forward(const megamoe_desc* desc, float swiglu_limit, const megam
 /* megamoe_mx_forward in one kernel launch (the reference's budget of one launch per call,
  * megabench/cases.py:32): one persistent kernel runs the permute, the expert units and the
  * combine, with the results of megamoe_mx_forward bit for bit. Rows that average 24 or more
- * per expert (12 or more where H*I is 8M and more), as the batch-shaped EP share's, take
- * megamoe_mx_forward's kernels instead. Workspace:
+ * per expert (where H*I is 8M and more, 12, or 13 below 14M with more than 64 experts), as the
+ * batch-shaped EP share's, take megamoe_mx_forward's kernels instead. Workspace:
  * megamoe_mx_workspace_bytes(desc) bytes, ZEROED before its first use with this entry point;
  * each call leaves its control words zero again. Calls sharing a workspace must be ordered.
  * `events` is NULL or events[0..1], recorded before and after the call. Replaces

@@ -42,3 +42,25 @@ def test_chunk_edges_equal_small_calls(counts, hidden, intermediate):
         want = experts(*part)
         torch.cuda.synchronize()
         assert torch.equal(got[max(0, min(r, R - step)):][:step], want), r
+
+
+@pytest.mark.parametrize("local,rows,batch", [(64, 8, True), (72, 12, False), (72, 13, True)])
+def test_many_experts_keep_the_decode_units_longer(local, rows, batch):
+    """Large experts (8M weights a matrix): 64 of them take the batch units from 8 rows an expert, more
+    of them from 13; the same bits as in calls of fewer rows."""
+    print(local, rows, flush=True)
+    case = replace(EPCASE, id="mx-many", gpus=1, ep=1,
+                   params=dict(tokens=local * rows, experts=local, topk=1, hidden=4096, intermediate=2048))
+    v = {k: t.to(DEV) for k, t in workloads.make_mx_inputs(workloads.serial_case(case), 31, DEV).items()}
+    ids = (torch.arange(local * rows) % local).to(DEV)
+    experts = EP.Experts(v["l1_blocks"], v["l1_scales"], v["l2_blocks"], v["l2_scales"], 0, case.swiglu_limit)
+    args = (v["x"], v["x_scales"], ids, v["topk_weights"].flatten())
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = experts(*args)
+        torch.cuda.synchronize()
+    assert any("k_experts_mx_batch" in e.name for e in prof.events()) == batch
+    step = 4 * local  # decode units
+    for r in range(0, local * rows - step + 1, step):
+        want = experts(*[a[r:r + step].contiguous() for a in args])
+        torch.cuda.synchronize()
+        assert torch.equal(got[r:r + step], want), r

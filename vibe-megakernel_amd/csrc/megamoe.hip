@@ -6262,20 +6262,25 @@ LayoutMx make_layout_mx(const megamoe_desc& d) {
 }
 
 // Whether the stream-ordered experts run as batch units (k_experts_mx_batch, one workgroup per CU) or
-// as decode units (two): from 24 rows an expert on average, and from 8 where the experts' weights are
-// large enough (8M per matrix and more) that the batch units' few long ones still balance. One call,
-// decode -> batch at 8 / 12 / 16 / 24 rows an expert: 48 experts of H 7168, I 3072 333 -> 322, 363 ->
-// 326, 383 -> 336, 369 -> 344 us (at 4: 299 -> 295); 96 of them 600 -> 600, 662 -> 626, 727 -> 634,
-// 703 -> 660 (at 4: 536 -> 572); 48 of 2048 by 2048 119 -> 129, 137 -> 132, 142 -> 136, 157 -> 146; 128
-// of 2048 by 1024 106 -> 132, 114 -> 135, 144 -> 159, 216 -> 201. Both give the same bits.
+// as decode units (two), by the rows an expert has on average. Experts of less than 8M weights a matrix:
+// from 24 rows (48 of 2048 by 2048 at 8 / 12 / 16 / 24 rows, decode -> batch: 119 -> 129, 137 -> 132, 142
+// -> 136, 157 -> 146 us; 128 of 2048 by 1024 106 -> 132, 114 -> 135, 144 -> 159, 216 -> 201). Larger ones:
+// from 8 rows up to 64 experts (at 8 / 12 rows, 48 of H 7168, I 3072 334 -> 323, 364 -> 325 us; at 8, 16 /
+// 32 / 64 of H 4096, I 2048 107 -> 82, 138 -> 118, 201 -> 193, and 72 of them 210 -> 214); of more experts
+// from 10 rows at 14M weights and more (at 8 / 10 / 12 rows, 128 of H 7168, I 2048 544 -> 564, 571 -> 573,
+// 592 -> 576 us, 256 of them 1114 -> 1137, 1171 -> 1161, 1225 -> 1173; 96 of H 7168, I 3072 605 -> 614, 644
+// -> 618, 673 -> 622) and from 13 below (at 8 / 12 / 13 rows, 72 of H 4096, I 2048 206 -> 211, 217 -> 215,
+// 222 -> 215; 128 of them 323 -> 355, 353 -> 359, 361 -> 363; 96 of H 5120, I 2048 313 -> 351, 343 -> 350,
+// 352 -> 352). Both give the same bits.
 //
 // `single`: for megamoe_mx_layer_forward, whose other form is one launch (k_layer_mx) that pays no
-// launch gaps: from 12 rows of large experts. k_layer_mx -> the three launches at 8 / 10 or 12 / 16 rows:
-// 48 experts of H 7168, I 3072 314 -> 322, 343 -> 325, 381 -> 329 us; 384 of them 2467 -> 2400, 2717 ->
-// 2470, 3010 -> 2575; 64 of H 4096, I 2048 187 -> 192, 200 -> 194, 220 -> 203.
+// launch gaps: from 12 rows of large experts at least. k_layer_mx -> the three launches at 8 / 10 or 12 /
+// 16 rows: 48 experts of H 7168, I 3072 314 -> 322, 343 -> 325, 381 -> 329 us; 384 of them 2467 -> 2400,
+// 2717 -> 2470, 3010 -> 2575; 64 of H 4096, I 2048 187 -> 192, 200 -> 194, 220 -> 203.
 bool batch_units_mx(const megamoe_desc& d, const LayoutMx& L, bool single) {
-  const bool large = (int64_t)d.hidden * d.intermediate >= ((int64_t)8 << 20);
-  const int rows = !large ? 24 : (single ? 12 : 8);
+  const int64_t weights = (int64_t)d.hidden * d.intermediate, M = (int64_t)1 << 20;
+  int rows = weights < 8 * M ? 24 : (d.experts <= 64 ? 8 : (weights >= 14 * M ? 10 : 13));
+  if (single && rows < 12) rows = 12;
   return (int64_t)d.tokens * d.topk >= (int64_t)rows * d.experts && (d.hidden / kMxStageK) % 2 == 0 &&
          (d.intermediate / kMxStageK / L.ks) % 2 == 0;
 }
