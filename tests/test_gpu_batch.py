@@ -60,6 +60,40 @@ def test_batch_units_equal_the_stream_ordered_kernels(case):
             assert torch.equal(a[k], b[k]), k
 
 
+def _few(tokens, experts, topk, batch, hidden=256, intermediate=256, act="fp8"):
+    return _case(MIXTRAL, act, tokens=tokens, experts=experts, topk=topk, hidden=hidden, intermediate=intermediate), batch
+
+
+@pytest.mark.parametrize("case,batch", [
+    # Both sides of each line: 12 rows from 208 tokens, 3 up to 64 experts, 8 from 512 tokens, 2 from
+    # 1024 and where the permute ranks in tiles (1024 experts from 449 tokens).
+    _few(208, 512, 1, False), _few(208, 512, 1, False, act="bf16"), _few(208, 128, 7, False), _few(208, 128, 8, True),
+    _few(207, 128, 8, False), _few(207, 64, 1, False), _few(208, 64, 1, True), _few(511, 128, 2, False),
+    _few(512, 128, 2, True), _few(1023, 256, 2, False), _few(1024, 256, 2, True), _few(448, 1024, 8, False),
+    _few(449, 1024, 8, True), _few(449, 1024, 4, False),
+    # Experts of 8M weights: 4.5 rows from 128 tokens, 2 from 512.
+    _few(128, 32, 1, False, 4096, 2048), _few(128, 32, 1, False, 4096, 2048, "bf16"), _few(143, 32, 1, False, 4096, 2048),
+    _few(144, 32, 1, True, 4096, 2048), _few(144, 32, 1, True, 4096, 2048, "bf16"),
+    _few(127, 16, 1, False, 2048, 4096), _few(128, 16, 1, True, 2048, 4096), _few(512, 256, 1, True, 8192, 1024),
+    _few(512, 257, 1, False, 8192, 1024),
+], ids=lambda v: f"t{v.tokens}-e{v.experts}-k{v.topk}-h{v.hidden}-{v.activations}" if isinstance(v, C.Case) else str(v))
+def test_each_side_of_the_batch_line(case, batch):
+    print(_id(case), flush=True)
+    one, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
+    values = workloads.make_inputs(case, 3, DEV)
+    one(values)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        a = one(values)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "k_" in e.name]
+    assert len(names) == 1 and ("k_layer_batch" in names[0]) == batch, names
+    b = five(values)
+    torch.cuda.synchronize()
+    for k in ("y", "expert_ids", "expert_weights"):
+        assert torch.equal(a[k], b[k]), k
+
+
 def test_batch_kernel_runs_and_is_one_launch():
     case = _case(DEEPSEEK, tokens=256)
     run = submission.MoELayer(case)

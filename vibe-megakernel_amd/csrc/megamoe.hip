@@ -5677,18 +5677,41 @@ bool split_gate_up(const megamoe_desc& d, int parts) {
 // stream an expert's weights more than once. The batch form also routes four tokens a unit, ranks
 // entries as they are routed and cuts the router into fewer splits, where the decode form's
 // front end grows with the tokens (the permute of 2048 x 8 entries in one workgroup: 219 us).
-// One call, decode -> batch: DeepSeek-V3's shape at 64 / 128 / 256 / 512 tokens 767 -> 788, 918 ->
-// 907, 1165 -> 1093, 1569 -> 1276 us (W8A16 788 -> 824, 985 -> 937, 1397 -> 1178, 2209 -> 1495),
-// Kimi-K2's at 128 (2.7 rows an expert) 2106 -> 2114, Mixtral's at 64 / 256 / 512 303 -> 277, 559 ->
-// 388, 908 -> 583; experts of few weights pay more for the one workgroup per CU:
-// Qwen3-30B-A3B's at 128 / 192 / 256 / 2048 149 -> 158, 161 -> 164, 181 -> 170, 754 -> 385. Depends on
-// the geometry only; both give the same bits (the separate gate and up units, whose K rotations
-// differ, keep their geometries).
+//
+// The rule is a least number of rows an expert, which falls as the tokens grow. One call, decode ->
+// batch, W8A8 (W8A16 in brackets):
+//   * 16 rows at any T: Mixtral's shape at 64 / 256 / 512 tokens 296 -> 274, 541 -> 386, 949 -> 641 us; 64
+//     experts of H 2048, I 1408 at 16 rows 146 -> 136 (156 -> 138), at 15 equal.
+//   * Experts of less than 8M weights a matrix, from 208 tokens 12 rows, or 3 up to 64 experts, from 512
+//     tokens 8: Qwen3-30B-A3B's shape (128 experts) at 208 / 256 / 512 / 2000 tokens 162 -> 161, 178 -> 167,
+//     228 -> 191, 617 -> 378, with top-4 at 8 / 12.5 / 16 rows 156 -> 164, 174 -> 168, 191 -> 174, with
+//     top-2 and 512 tokens 165 -> 166 (170 -> 162); 512 experts of H 2048, I 512 at 5 / 8 / 10 rows 350 -> 380,
+//     384 -> 394, 409 -> 397; 64 of I 768 at 3.3 / 6.3 rows 95 -> 94, 110 -> 99.
+//   * From 1024 tokens 2 rows: 1024 experts of H 2048, I 512, top-2, 745 -> 700 (756 -> 746), 512 of H 4096,
+//     I 1024, top-1, 1069 -> 1033 (1093 -> 1091); and where the decode form's permute ranks in tiles, its
+//     bitmaps not fitting the LDS (1024 experts, top-8, 400 / 480 tokens 647 -> 688, 803 -> 712).
+//   * Larger experts, from 128 tokens 4.5 rows, from 512 tokens 2. What 4 to 6 rows give depends on how
+//     even the routing is, which the host does not know; the line lies where the sum over the three
+//     routings below changes sides. DeepSeek-V3's shape at 4 / 4.5 / 5 / 6.5 / 8 rows, correction bias of
+//     std 0.1 981 -> 975, 1011 -> 990, 1057 -> 1028, 1123 -> 1074, 1184 -> 1114 (1048 -> 1022, 1096 -> 1047,
+//     1150 -> 1083, 1292 -> 1150, 1423 -> 1206), of std 0.03 1490 -> 1508, 1530 -> 1535, 1553 -> 1553, 1673 ->
+//     1653, 1728 -> 1681 (1544 -> 1604, 1590 -> 1627, 1622 -> 1662, 1770 -> 1763, 1858 -> 1795), without one
+//     1702 -> 1727, 1747 -> 1754, 1765 -> 1769, 1800 -> 1788, 1835 -> 1805 (1757 -> 1874, 1806 -> 1908, 1816 ->
+//     1890, 1883 -> 1913, 1942 -> 1932). Kimi-K2's at 4 rows 2325 -> 2331 (2465 -> 2487), GLM-5.3-Flash's at
+//     4 / 5 / 7 / 14 rows 666 -> 657, 705 -> 684, 764 -> 725, 1024 -> 875. DeepSeek-V3's with top-1 and no bias
+//     at 1 / 2 rows 1157 -> 1174, 1574 -> 1549.
+// Depends on the geometry only; both give the same bits (the separate gate and up units, whose K
+// rotations differ, keep their geometries).
 bool batch_units(const megamoe_desc& d) {
-  const int64_t entries = (int64_t)d.tokens * d.topk, E = d.experts;
+  const int64_t T = d.tokens, E = d.experts, entries = T * d.topk;
   const bool large = (int64_t)d.hidden * d.intermediate >= ((int64_t)8 << 20);
-  return !dense_experts(d) && d.hidden % (2 * kBlock) == 0 &&
-         (d.tokens >= 208 || entries >= 16 * E || (large && d.tokens >= 128 && entries >= 4 * E));
+  const bool tiled = permute_tile_waves(d.tokens, d.experts, 256, kPermuteLdsInts) > 0;
+  int64_t rows2 = 32;  // the least rows an expert, doubled
+  if (large)
+    rows2 = T >= 512 ? 4 : (T >= 128 ? 9 : 32);
+  else if (T >= 208)
+    rows2 = T >= 1024 || tiled ? 4 : (E <= 64 ? 6 : (T >= 512 ? 16 : 24));
+  return !dense_experts(d) && d.hidden % (2 * kBlock) == 0 && 2 * entries >= rows2 * E;
 }
 
 Layout layout_with(const megamoe_desc& d, int parts) {
