@@ -3074,6 +3074,7 @@ struct DownArgs {
   int T, H, I, K, S, E, ks;
   int dense;      // the dense schedule: units from dense_dn_chunk, rows e*T + t
   int rows_r;     // routed rows of d_r and of each part of p_r: T*K, or E*T in the dense schedule
+  int keyed;      // the K rotation by weight block (a geometry of the batch form), not by unit
   const uint16_t* h16_r;  // W8A16: bf16 h of the routed rows [rows_r, I]
   const uint16_t* h16_s;  // W8A16: of the shared rows [T, S*I]
 };
@@ -3175,7 +3176,8 @@ __device__ __forceinline__ void down_work(const DownArgs& a, int v, const ReadyW
   const int c = v / (nbH * a.ks);
   const int4 ch = a.dense ? dense_dn_chunk(c, a.E, a.S, a.T) : a.chunks[c];
   const int rem = v % (nbH * a.ks), j = rem / a.ks, kp = rem % a.ks;
-  const int rot = down_rotation(ch.x, j >> 1, kp, a.H, a.I, a.ks);
+  // Concurrent units start at different K blocks, keyed as gateup_work's.
+  const int rot = a.keyed ? down_rotation(ch.x, j >> 1, kp, a.H, a.I, a.ks) : v % (nbI / a.ks);
   float* pd_s = a.p_s + (size_t)kp * a.T * a.H;
   float* pd_r = a.p_r + (size_t)kp * a.rows_r * a.H;
   if (ch.x == a.E) {
@@ -5626,8 +5628,9 @@ int down_splits(const megamoe_desc& d) {
 // from the moment the routing is known; those started before stream weights no combine
 // reads, which the roofline's algorithmic bytes do not count. Each routed row's bits are the
 // routed schedule's (each MFMA output column depends only on its own row); only the K
-// rotation of a unit, keyed by its place in the lists, differs, and both forms (single
-// launch and stream-ordered) take the same lists. Depends on the geometry only.
+// rotation of a whole-block gate/up unit and of a down unit, keyed by its place in the lists,
+// differs, and both forms (single launch and stream-ordered) take the same lists. Depends on the
+// geometry only.
 bool dense_experts(const megamoe_desc& d) {
   return d.tokens <= 16 && (int64_t)d.tokens * d.topk >= d.experts;
 }
@@ -5994,6 +5997,7 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   da.T = T; da.H = H; da.I = I; da.K = K; da.S = S; da.E = E;
   da.dense = L.dense;
   da.rows_r = L.rows_r;
+  da.keyed = batch_units(d) ? 1 : 0;
   da.h16_r = ga.h16_r;
   da.h16_s = ga.h16_s;
   ea.dn_of_gu = po.dn_of_gu;
