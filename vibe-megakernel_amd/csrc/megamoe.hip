@@ -6153,13 +6153,16 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   la.gate = d.gate; la.renorm = d.renormalize; la.pow2 = d.pow2_scales;
   la.nsplit = L.nsplit;
   la.n_et = (E + kRouterTile - 1) / kRouterTile;
+  const bool split = !a16 && L.split;
+  const bool batch = !split && batch_units(d);
+  const size_t resident = (size_t)di.cus * (batch ? 1 : di.layer_per_cu);  // workgroups at once
   const int tiles = (T + kRouterTile - 1) / kRouterTile;
   // Token tiles per router unit: k_router's choice, halved while the units still fit in one
-  // round of the grid (a shorter fp64 MFMA chain per unit: Qwen3-30B-A3B 139 -> 136 us).
+  // round of the resident workgroups (a shorter fp64 MFMA chain per unit: Qwen3-30B-A3B's shape at 32
+  // tokens 139 -> 136 us; in the batch form, whose one workgroup per CU makes a round half as many
+  // units, counting two made it 161 -> 164, 165 -> 168 at 208 and 256 tokens).
   la.ntt = tiles <= 1 ? 1 : (tiles <= 2 ? 2 : 4);
-  while (la.ntt > 1 && (size_t)la.n_et * L.nsplit * ((tiles + la.ntt / 2 - 1) / (la.ntt / 2)) <=
-                           (size_t)di.cus * di.layer_per_cu)
-    la.ntt /= 2;
+  while (la.ntt > 1 && (size_t)la.n_et * L.nsplit * ((tiles + la.ntt / 2 - 1) / (la.ntt / 2)) <= resident) la.ntt /= 2;
   const int passes = (tiles + la.ntt - 1) / la.ntt;
   la.vpl = E <= 64 ? 1 : (E <= 128 ? 2 : (E <= 256 ? 4 : (E <= 512 ? 8 : 16)));
   la.ks = L.ks;
@@ -6170,8 +6173,6 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
 
   // As many workgroups as fit on the device at once, and no more than the most units the
   // queue can hold.
-  const bool split = !a16 && L.split;
-  const bool batch = !split && batch_units(d);
   const int parts = L.parts;
   const size_t units_max = (size_t)la.n_norm + la.n_router + T +
                            expert_units_max(d, L, split ? 2 : parts, a16 ? kChunkRowsA16 : kChunkRows) +
@@ -6185,7 +6186,6 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   if (L.dense) la.ex.ready = (int*)(ws + L.ready_l);
   if (L.n_pairs_l) la.ex.gu.pairs = (int*)(ws + L.pairs_l);
   la.n_pairs = L.n_pairs_l;
-  const size_t resident = (size_t)di.cus * (batch ? 1 : di.layer_per_cu);
   const unsigned grid = (unsigned)(units_max < resident ? units_max : resident);
   // Router units taken by workgroup index: the first round of them, when there are 64 or more
   // (fewer are claimed from the queue in ~1 us: Mixtral's 8 measured 2 us slower by index);
