@@ -386,16 +386,28 @@ inline int router_splits(int H) {
   return best;
 }
 
-// At batch sizes (batch_units) there are token passes enough to fill the chip: the splits halve
-// while the units exceed kRouterBatchUnits, so each unit's MFMA chain runs over more channels
-// (its start, sums and stores counted less often) and the routing adds fewer partials (16 splits of
-// 512 x 256 logits are 17 MB in fp64).
-constexpr int kRouterBatchUnits = 512;
+// At batch sizes (batch_units) there are token passes enough to fill the chip: fewer splits, whose
+// units' MFMA chains run over more channels (their start, sums and stores counted less often) and which
+// leave the routing fewer partials to add (16 splits of 512 x 256 logits are 17 MB in fp64). The number
+// whose units take the least time in rounds of a reference grid, one workgroup per CU on 256 CUs, a
+// unit costing 1/n of the channels and a tenth for itself. Against halving while the units exceed 512
+// (two rounds, and 288 units of GLM-5.3-Flash's 512 tokens in one and an eighth): DeepSeek-V3's shape at 512
+// tokens 1340 -> 1321 us, Qwen3-30B-A3B's at 2000 373 -> 367, GLM-5.3-Flash's at 512 873 -> 866 (stream-ordered
+// 1015 -> 1006). Depends on the geometry only; the router's partial sums are fp64 in either number.
+constexpr int kRouterGrid = 256;
 inline int router_splits_batch(int H, int E, int T) {
-  int n = router_splits(H);
-  const int tiles = (T + kRouterTile - 1) / kRouterTile, passes = (tiles + 3) / 4;
-  while (n > 1 && (int64_t)n * ((E + kRouterTile - 1) / kRouterTile) * passes > kRouterBatchUnits) n /= 2;
-  return n;
+  const int most = router_splits(H), tiles = (T + kRouterTile - 1) / kRouterTile;
+  const int64_t units = (int64_t)((E + kRouterTile - 1) / kRouterTile) * ((tiles + 3) / 4);  // of one split
+  int best = most;
+  double least = 0.0;
+  for (int n = most; n >= 1; n /= 2) {
+    const double cost = (double)((units * n + kRouterGrid - 1) / kRouterGrid) * (1.0 / n + 0.1);
+    if (n == most || cost <= least) {
+      best = n;
+      least = cost;
+    }
+  }
+  return best;
 }
 
 inline int router_quant_groups(int T, int H) {
