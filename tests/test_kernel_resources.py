@@ -30,6 +30,8 @@ STREAM_KERNELS = [
     "(anonymous namespace)::k_experts<false, false>",
     "(anonymous namespace)::k_experts<true, false>",
     "(anonymous namespace)::k_experts<false, true>",  # the W8A16 form
+    "(anonymous namespace)::k_experts_small<false>",
+    "(anonymous namespace)::k_experts_small<true>",
     "(anonymous namespace)::k_experts_mx",
     "(anonymous namespace)::k_experts_mx_batch",
 ]
@@ -39,8 +41,14 @@ STREAM_KERNELS = [
 def test_expert_stream_kernels_have_no_scratch(kernel):
     r = _entry(_report(), kernel)
     assert r["scratch_bytes"] == 0 and r["vgpr_spills"] == 0, (kernel, r)
-    # Two workgroups of 256 threads per CU (k_experts_mx_batch: one, with its LDS rings).
-    assert r["occupancy"] >= (1 if kernel.endswith("_batch") else 2), (kernel, r)
+    _fits(kernel, r)
+
+
+def _fits(kernel, r):
+    """Two workgroups of 256 threads per CU (the batch kernels: one, with their LDS rings), by the
+    registers and by the 160 KB of LDS; the launches size their grids for that."""
+    per_cu = 1 if "_batch" in kernel else 2
+    assert r["occupancy"] >= per_cu and r["lds_bytes"] * per_cu <= 160 << 10, (kernel, r)
 
 
 # The single-launch kernels hold the front end (norm, router, routing, permute) and the
@@ -48,11 +56,16 @@ def test_expert_stream_kernels_have_no_scratch(kernel):
 # register file. None of them spills a VGPR: the routing keeps its logits, choices and bias in
 # LDS (and, from 512 experts, its selection keys), derives its expert indices from an opaque
 # lane so they are not hoisted out of the persistent loop, and the combine takes its first
-# slots by value. k_layer<false, ...> keeps a 20-byte private segment that no instruction uses.
+# slots by value. k_layer<false, ...> and k_layer_small<false> keep a 20-byte private segment that no
+# instruction uses.
 LAYER_CEILINGS = {
     "(anonymous namespace)::k_layer<false, false>": {"vgpr_spills": 0, "scratch_bytes": 20},
     "(anonymous namespace)::k_layer<true, false>": {"vgpr_spills": 0, "scratch_bytes": 20},
     "(anonymous namespace)::k_layer<false, true>": {"vgpr_spills": 0, "scratch_bytes": 20},  # the W8A16 form
+    "(anonymous namespace)::k_layer_small<false>": {"vgpr_spills": 0, "scratch_bytes": 20},
+    "(anonymous namespace)::k_layer_small<true>": {"vgpr_spills": 0, "scratch_bytes": 20},
+    "(anonymous namespace)::k_layer_batch<false>": {"vgpr_spills": 0, "scratch_bytes": 0},
+    "(anonymous namespace)::k_layer_batch<true>": {"vgpr_spills": 0, "scratch_bytes": 0},
     "(anonymous namespace)::k_layer_mx": {"vgpr_spills": 0, "scratch_bytes": 0},
 }
 
@@ -70,7 +83,16 @@ def test_single_launch_kernels_spill_no_more_than_now(kernel):
     r = _entry(_report(), kernel)
     for field, ceiling in LAYER_CEILINGS[kernel].items():
         assert r[field] <= ceiling, (kernel, field, r)
-    assert r["occupancy"] >= 2, (kernel, r)
+    _fits(kernel, r)
+
+
+def test_every_expert_and_layer_kernel_is_checked():
+    names = _demangle(list(_report()))
+    listed = [*STREAM_KERNELS, *LAYER_CEILINGS]
+    for d in names:
+        name = d.removeprefix("void ").split("(anonymous namespace)::", 1)[-1].split("(")[0]
+        if name.startswith(("k_experts", "k_layer")):
+            assert f"(anonymous namespace)::{name}" in listed, name
 
 
 def test_parser_reads_hipcc_remarks():

@@ -5835,12 +5835,23 @@ int validate(const megamoe_desc* d) {
 
 struct DeviceInfo {
   int cus = 0;
-  int experts_per_cu = 0;     // resident k_experts workgroups per CU
-  int experts_mx_per_cu = 0;  // resident k_experts_mx workgroups per CU
-  int batch_mx_per_cu = 0;    // resident k_experts_mx_batch workgroups per CU
-  int layer_per_cu = 0;       // resident k_layer workgroups per CU
-  int layer_mx_per_cu = 0;    // resident k_layer_mx workgroups per CU
+  int experts_per_cu = 0;     // resident workgroups per CU of k_experts and k_experts_small
+  int experts_mx_per_cu = 0;  // of k_experts_mx
+  int batch_mx_per_cu = 0;    // of k_experts_mx_batch
+  int layer_per_cu = 0;       // of k_layer and k_layer_small
+  int layer_batch_per_cu = 0; // of k_layer_batch
+  int layer_mx_per_cu = 0;    // of k_layer_mx
 };
+
+// Lowers *per_cu (0: not set yet) to the resident workgroups per CU of a kernel of 256 threads.
+template <class Kernel>
+bool fit_per_cu(int* per_cu, Kernel kernel) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 256, 0) != hipSuccess) return false;
+  n = n > 0 ? n : 1;
+  if (*per_cu == 0 || n < *per_cu) *per_cu = n;
+  return true;
+}
 
 // The figures of the current device, queried on its first call and kept per device. The
 // mutex covers the fill: two host threads making their first calls at once must not see a
@@ -5854,29 +5865,19 @@ int device_info(DeviceInfo* out) {
   DeviceInfo& di = cache[dev];
   if (di.cus == 0) {
     DeviceInfo fill;
-    int cus = 0, per_cu = 0;
+    int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return MEGAMOE_ERR_HIP;
-    int per_cu_split = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_experts<false>, 256, 0) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_split, k_experts<true>, 256, 0) != hipSuccess)
+    if (!fit_per_cu(&fill.experts_per_cu, k_experts<false>) || !fit_per_cu(&fill.experts_per_cu, k_experts<true>) ||
+        !fit_per_cu(&fill.experts_per_cu, k_experts<false, true>) ||
+        !fit_per_cu(&fill.experts_per_cu, k_experts_small<false>) ||
+        !fit_per_cu(&fill.experts_per_cu, k_experts_small<true>) ||
+        !fit_per_cu(&fill.experts_mx_per_cu, k_experts_mx) || !fit_per_cu(&fill.batch_mx_per_cu, k_experts_mx_batch) ||
+        !fit_per_cu(&fill.layer_per_cu, k_layer<false>) || !fit_per_cu(&fill.layer_per_cu, k_layer<true>) ||
+        !fit_per_cu(&fill.layer_per_cu, k_layer<false, true>) || !fit_per_cu(&fill.layer_per_cu, k_layer_small<false>) ||
+        !fit_per_cu(&fill.layer_per_cu, k_layer_small<true>) ||
+        !fit_per_cu(&fill.layer_batch_per_cu, k_layer_batch<false>) ||
+        !fit_per_cu(&fill.layer_batch_per_cu, k_layer_batch<true>) || !fit_per_cu(&fill.layer_mx_per_cu, k_layer_mx))
       return MEGAMOE_ERR_HIP;
-    per_cu = per_cu_split < per_cu ? per_cu_split : per_cu;
-    fill.experts_per_cu = per_cu > 0 ? per_cu : 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_experts_mx, 256, 0) != hipSuccess)
-      return MEGAMOE_ERR_HIP;
-    fill.experts_mx_per_cu = per_cu > 0 ? per_cu : 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_experts_mx_batch, 256, 0) != hipSuccess)
-      return MEGAMOE_ERR_HIP;
-    fill.batch_mx_per_cu = per_cu > 0 ? per_cu : 1;
-    int per_cu_split2 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_layer<false>, 256, 0) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_split2, k_layer<true>, 256, 0) != hipSuccess)
-      return MEGAMOE_ERR_HIP;
-    per_cu = per_cu_split2 < per_cu ? per_cu_split2 : per_cu;
-    fill.layer_per_cu = per_cu > 0 ? per_cu : 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_layer_mx, 256, 0) != hipSuccess)
-      return MEGAMOE_ERR_HIP;
-    fill.layer_mx_per_cu = per_cu > 0 ? per_cu : 1;
     fill.cus = cus > 0 ? cus : 1;
     di = fill;
   }
@@ -6167,7 +6168,7 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   la.n_et = (E + kRouterTile - 1) / kRouterTile;
   const bool split = !a16 && L.split;
   const bool batch = !split && batch_units(d);
-  const size_t resident = (size_t)di.cus * (batch ? 1 : di.layer_per_cu);  // workgroups at once
+  const size_t resident = (size_t)di.cus * (batch ? di.layer_batch_per_cu : di.layer_per_cu);  // workgroups at once
   const int tiles = (T + kRouterTile - 1) / kRouterTile;
   // Token tiles per router unit: k_router's choice, halved while the units still fit in one
   // round of the resident workgroups (a shorter fp64 MFMA chain per unit: Qwen3-30B-A3B's shape at 32
