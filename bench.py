@@ -13,9 +13,9 @@ independent input sets as it takes to move >= 1 GB per rotation, so the 256 MB
 Infinity Cache cannot hold a step's weights.
 
 Printed: one JSON line (rank 0) with the headline metric of the DeepSeek-V3
-shape (or --case), the roofline of the dominant kernel (k_experts<false|true>:
-gate/up + SwiGLU + down; k_experts_mx for the MXFP4 forms) and the CPU oracle timed on a
-bounded sample. Without --case, the line's "configs" also holds the other four
+shape (or --case), the roofline of the single launch (the kernel layer_kernel names; for
+the stream-ordered form and the EP share the expert kernel, expert_kernel) and the CPU oracle
+timed on a bounded sample. Without --case, the line's "configs" also holds the other four
 BASELINE.json configs, each measured the same way (time, p50/p95, TB/s, roofline, its
 own CPU baseline) in a child process; --all adds the other forms (the block forms, the
 MXFP4 layer, rank 0's EP share, the epilogue variants). For an EP case a step is rank 0's
@@ -85,38 +85,87 @@ def kernel_bytes(case, hit: int) -> dict:
     return {"gate_up": gu, "down": dn}
 
 
-def mx_kernel(rows: int, experts: int) -> str:
-    """The MXFP4 expert kernel of the stream-ordered form: batch mode from 24 rows per expert
-    on average (kBatchMinRows in the library), the decode kernel below."""
-    return "k_experts_mx_batch" if rows >= 24 * experts else "k_experts_mx"
+# The library picks a kernel by the geometry (csrc/megamoe.hip); the functions below name its pick, and
+# tests/test_gpu_bench_labels.py holds them to the kernels that run.
+
+
+def _dense(case) -> bool:
+    """dense_experts: every expert's units over all tokens, in lists known from the geometry."""
+    return case.tokens <= 16 and case.tokens * case.topk >= case.experts
+
+
+def _parts(case) -> int:
+    """small_parts_wanted: the small form's units per 128-row block of gate and up (1: whole blocks)."""
+    nkb, block_bytes = case.hidden // 128, 2 * 128 * case.hidden
+    blocks = (min(case.experts, case.tokens * case.topk) + case.shared_experts) * (case.intermediate // 128)
+    if case.tokens > 16 or (_dense(case) and block_bytes < 512 << 10):
+        return 1
+    p = 1
+    while p < 8 and nkb % p == 0 and (blocks * p < (1024 if block_bytes // p >= 256 << 10 else 512)
+                                      or (blocks * p < 2048 and block_bytes // (2 * p) >= 512 << 10)):
+        p *= 2
+    return p
 
 
 def _split(case) -> bool:
-    """split_gate_up in csrc/megamoe.hip: the split gate/up form when the whole-block gate/up
-    units cannot fill one round of a 512-workgroup grid with every expert hit and the rows
-    have 32 or more K blocks (never in the W8A16 form)."""
+    """split_gate_up: the split gate/up form when the whole-block gate/up units cannot fill one
+    round of a 512-workgroup grid with every expert hit and the rows have 32 or more K blocks
+    (never in the W8A16 form, the dense schedule or the small form)."""
     hit = min(case.experts, case.tokens * case.topk) + case.shared_experts
-    return case.activations != "bf16" and hit * (case.intermediate // 128) < 512 and case.hidden // 128 >= 32
+    return (case.activations != "bf16" and not _dense(case) and _parts(case) == 1
+            and hit * (case.intermediate // 128) < 512 and case.hidden // 128 >= 32)
 
 
-def fp8_kernel(case) -> str:
-    """The FP8 expert kernel the library runs (k_experts<split, w8a16>)."""
-    return f"k_experts<{str(_split(case)).lower()}, {str(case.activations == 'bf16').lower()}>"
+def _batch(case) -> bool:
+    """batch_units: a least number of rows an expert, which falls as the tokens grow."""
+    T, E, entries = case.tokens, case.experts, case.tokens * case.topk
+    tiled = E * (1 + (T + 31) // 32) + 32 > 16384  # the decode form's permute
+    rows = 16.0
+    if case.hidden * case.intermediate >= 8 << 20:
+        rows = 2.0 if T >= 512 else 4.5 if T >= 128 else 16.0
+    elif T >= 208:
+        rows = 2.0 if T >= 1024 or tiled else 3.0 if E <= 64 else 8.0 if T >= 512 else 12.0
+    return not _dense(case) and case.hidden % 256 == 0 and entries >= rows * E
+
+
+def mx_kernel(case, rows: int, experts: int, single: bool = False) -> str:
+    """The MXFP4 expert kernel for `rows` rows over `experts` experts (batch_units_mx; `single`:
+    below the single launch, which is k_layer_mx where this names k_experts_mx)."""
+    weights, M = case.hidden * case.intermediate, 1 << 20
+    least = 24 if weights < 8 * M else 8 if experts <= 64 else 10 if weights >= 14 * M else 13
+    if single:
+        least = max(least, 12)
+    units, stages, ks = min(experts, rows) * (case.hidden // 128), case.intermediate // 256, 1
+    while ks < 8 and units * ks < 2048 and stages % (2 * ks) == 0:
+        ks *= 2
+    batch = rows >= least * experts and case.hidden // 256 % 2 == 0 and stages // ks % 2 == 0
+    return "k_experts_mx_batch" if batch else "k_experts_mx"
+
+
+def _form(case) -> str:
+    return str(case.activations == "bf16").lower()
 
 
 def expert_kernel(case) -> str:
     """The expert kernel of the stream-ordered form."""
     if case.format == "mxfp4":
-        return mx_kernel(case.tokens * case.topk, case.experts)
-    return fp8_kernel(case)
+        return mx_kernel(case, case.tokens * case.topk, case.experts)
+    if _parts(case) > 1:
+        return f"k_experts_small<{_form(case)}>"
+    return f"k_experts<{str(_split(case)).lower()}, {_form(case)}>"
 
 
 def layer_kernel(case) -> str:
-    """The single-launch kernel: k_layer for the fp8 forms (split gate/up as fp8_kernel),
-    k_layer_mx for the MXFP4 form."""
+    """The single-launch kernel: for the fp8 forms k_layer_small, k_layer_batch or k_layer<split,
+    w8a16>; for the MXFP4 form k_layer_mx, or the expert kernel of the launches it becomes."""
     if case.format == "mxfp4":
-        return "k_layer_mx"
-    return f"k_layer<{str(_split(case)).lower()}, {str(case.activations == 'bf16').lower()}>"
+        kernel = mx_kernel(case, case.tokens * case.topk, case.experts, single=True)
+        return "k_layer_mx" if kernel == "k_experts_mx" else kernel
+    if _parts(case) > 1:
+        return f"k_layer_small<{_form(case)}>"
+    if _batch(case) and not _split(case):
+        return f"k_layer_batch<{_form(case)}>"
+    return f"k_layer<{str(_split(case)).lower()}, {_form(case)}>"
 
 
 def measured_traffic(case, kernel: str = "k_experts") -> float | None:
@@ -576,8 +625,8 @@ def bench_ep_share(case, steps: int, warmup: int, want_cpu: bool, cpu_budget: fl
         "rotation_sets": 1, "received_rows": R, "sent_rows": T * K,
         "roofline": {"bound": "hbm", "achieved": ex_bytes / (ex_ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9,
                      "unit": "GB/s", "frac": ex_bytes / (ex_ms * 1e-3) / PEAK_HBM,
-                     "traffic": measured_traffic(case, mx_kernel(R, local)),
-                     "kernel": mx_kernel(R, local), "kernel_us": ex_ms * 1e3, "bytes_per_launch": ex_bytes},
+                     "traffic": measured_traffic(case, mx_kernel(case, R, local)),
+                     "kernel": mx_kernel(case, R, local), "kernel_us": ex_ms * 1e3, "bytes_per_launch": ex_bytes},
         "dtype": "e2m1xe4m3->fp32 (E8M0 scales per 32; bf16 out)",
     }
     if want_cpu:
