@@ -1,8 +1,8 @@
 """The single launch's batch units (k_layer_batch) against the stream-ordered kernels, whose decode
 units compute the same sums: bit for bit at chunk sizes around the units' tiles (32, 64 and 128
 rows and their remainders, more than one chunk an expert, experts no token picks), for both
-activation forms, with a shared expert of several chunks, K parts and the block steps; and
-against the CPU oracle once per form."""
+activation forms, with a shared expert of several chunks, 2, 4 and 8 K parts of the down units and
+the block steps; and against the CPU oracle once per form."""
 
 from __future__ import annotations
 
@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from oracle import layer, metrics
+from tests.down_parts import down_parts
 from vibe_megakernel_amd import cases as C
 from vibe_megakernel_amd import submission, workloads
 
@@ -31,7 +32,7 @@ def _cases():
         # Every token picks both experts: each holds `tokens` rows.
         out += [_case(MIXTRAL, act, tokens=t, experts=2, topk=2) for t in (17, 32, 33, 64, 65, 96, 128, 129, 257)]
         # Ragged rows per expert; one K block a row of h; an odd number of K blocks; rows of H = 4096
-        # (W8A8: gate and up apart, in both forms); K parts of the down units.
+        # (W8A8: gate and up apart, in both forms).
         out.append(_case(MIXTRAL, act, tokens=200, experts=8, intermediate=128))
         out.append(_case(MIXTRAL, act, tokens=300, experts=16, topk=3, hidden=768, intermediate=384))
         out.append(_case(MIXTRAL, act, tokens=70, experts=8, hidden=4096, intermediate=512))
@@ -47,8 +48,7 @@ def _id(c):
     return f"{c.model.split('/')[-1].split()[0]}-{c.activations}-t{c.tokens}-e{c.experts}-h{c.hidden}-i{c.intermediate}"
 
 
-@pytest.mark.parametrize("case", _cases(), ids=_id)
-def test_batch_units_equal_the_stream_ordered_kernels(case):
+def _equal_to_stream_ordered(case, kernel="k_layer_batch"):
     print(_id(case), flush=True)
     one, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
     for seed in (3, 4):  # consecutive calls on one workspace
@@ -58,6 +58,38 @@ def test_batch_units_equal_the_stream_ordered_kernels(case):
         assert not one.gave_up(torch.device(DEV))
         for k in ("y", "expert_ids", "expert_weights"):
             assert torch.equal(a[k], b[k]), k
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        one(values)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "k_" in e.name]
+    assert len(names) == 1 and kernel in names[0], names
+    return {k: v.cpu() for k, v in values.items()}, a
+
+
+@pytest.mark.parametrize("case", _cases(), ids=_id)
+def test_batch_units_equal_the_stream_ordered_kernels(case):
+    _equal_to_stream_ordered(case, "k_layer<true" if case.activations == "fp8" and case.hidden == 4096 else "k_layer_batch")
+
+
+def _part_cases():
+    # 16, 32 and 64 K blocks a row of h: 2, 4 and 8 parts of eight. Chunks of up to 32, 64 and 128 rows
+    # and more than one; a shared expert (parts of its own h rows, S*I wide), twice as wide in the last.
+    for act in ("fp8", "bf16"):
+        for parts, intermediate in ((2, 2048), (4, 4096), (8, 8192)):
+            yield parts, _case(MIXTRAL, act, tokens=20, experts=2, topk=2, intermediate=intermediate)
+            yield parts, _case(MIXTRAL, act, tokens=131, experts=4, topk=2, hidden=512, intermediate=intermediate)
+            yield parts, _case(DEEPSEEK, act, tokens=70, experts=8, hidden=512, intermediate=intermediate)
+        yield 2, replace(_case(DEEPSEEK, act, tokens=40, experts=8, intermediate=2048, shared_experts=2),
+                         norm="fp32_weight", residual=True)
+
+
+@pytest.mark.parametrize("parts,case", list(_part_cases()), ids=lambda v: _id(v) if isinstance(v, C.Case) else f"ks{v}")
+def test_batch_units_with_k_parts(parts, case):
+    assert down_parts(case) == parts
+    host, got = _equal_to_stream_ordered(case)
+    if case.tokens == 20:
+        check = metrics.layer_checks(got["y"], layer.reference(case, host)["y"])  # max-rel 1e-2, cosine 0.9999
+        assert check["pass"], check
 
 
 def _few(tokens, experts, topk, batch, hidden=256, intermediate=256, act="fp8"):

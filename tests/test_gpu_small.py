@@ -1,7 +1,8 @@
 """The small form (k_layer_small, k_experts_small: 2, 4 or 8 units per 128-row block of gate and up, at
 up to 16 tokens): the single launch against the stream-ordered kernels, bit for bit, for each number of
 parts the geometry allows, both activation forms, 0 to 2 shared experts, the dense schedule (with experts
-the routing leaves unpicked) and the routed one; and both against the CPU oracle."""
+the routing leaves unpicked) and the routed one, 2, 4 and 8 K parts of the down units; and both against
+the CPU oracle."""
 
 from __future__ import annotations
 
@@ -10,7 +11,9 @@ from dataclasses import replace
 import pytest
 import torch
 
+import bench
 from oracle import layer, metrics
+from tests.down_parts import down_parts
 from vibe_megakernel_amd import cases as C
 from vibe_megakernel_amd import submission, workloads
 
@@ -34,8 +37,10 @@ def _cases():
         # Dense: blocks of 512 KB and more; 17, 18 and 20 K blocks allow 2, 4 and 8 parts.
         out += [_case(MIXTRAL, act, tokens=t, experts=8, hidden=h) for t, h in ((4, 2176), (5, 2304), (16, 2560))]
         out.append(_case(DEEPSEEK, act, tokens=15, experts=32, topk=4, hidden=2048, shared_experts=2))
-        out.append(replace(_case(KIMI, act, tokens=12), norm="fp32_weight", residual=True))
-    out.append(replace(_case(DEEPSEEK, tokens=4, experts=16), swiglu="bf16", swiglu_limit=0.5, power_of_two=True))
+        out.append(replace(_case(KIMI, act, tokens=12), norm="fp32_weight", residual=True))  # dense: whole blocks
+        out.append(replace(_case(KIMI, act, tokens=12, experts=64), norm="fp32_weight", residual=True))
+    for experts in (16, 64):  # dense: whole blocks; routed: parts
+        out.append(replace(_case(DEEPSEEK, tokens=4, experts=experts), swiglu="bf16", swiglu_limit=0.5, power_of_two=True))
     return out
 
 
@@ -44,8 +49,7 @@ def _id(c):
             f"-s{c.shared_experts}")
 
 
-@pytest.mark.parametrize("case", _cases(), ids=_id)
-def test_small_units_equal_the_stream_ordered_kernels_and_the_oracle(case):
+def _check(case):
     print(_id(case), flush=True)
     one, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
     for seed in (3, 4):  # consecutive calls on one workspace
@@ -59,6 +63,43 @@ def test_small_units_equal_the_stream_ordered_kernels_and_the_oracle(case):
     want = layer.block_reference(case, host) if case.residual else layer.reference(case, host)
     check = metrics.layer_checks(a["y"], want["y"])  # the layer's bars: max-rel 1e-2, cosine 0.9999
     assert torch.equal(a["expert_ids"].cpu(), want["expert_ids"]) and check["pass"], check
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        one(values)
+        five(values)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events()]
+    for kernel in (bench.layer_kernel(case), bench.expert_kernel(case)):
+        assert ("_small<" in kernel) == (bench._parts(case) > 1) and any(f"::{kernel}(" in n or f" {kernel}(" in n
+                                                                         for n in names), (kernel, names)
+
+
+@pytest.mark.parametrize("case", _cases(), ids=_id)
+def test_small_units_equal_the_stream_ordered_kernels_and_the_oracle(case):
+    _check(case)
+
+
+def test_the_cases_have_every_number_of_units_a_block():
+    for act in ("fp8", "bf16"):
+        for dense in (False, True):
+            got = {bench._parts(c) for c in _cases() if c.activations == act and bench._dense(c) == dense}
+            assert got >= {2, 4, 8}, (act, dense, got)
+
+
+def _part_cases():
+    # Down units of 2, 4 and 8 K parts under both schedules, with and without a shared expert.
+    for act in ("fp8", "bf16"):
+        for parts, intermediate in ((2, 2048), (4, 4096), (8, 8192)):
+            yield parts, _case(MIXTRAL, act, tokens=1, experts=16, hidden=512, intermediate=intermediate)
+            yield parts, _case(DEEPSEEK, act, tokens=2, experts=16, topk=2, hidden=512, intermediate=intermediate)
+        yield 2, _case(DEEPSEEK, act, tokens=3, experts=16, topk=2, hidden=512, intermediate=2048, shared_experts=2)
+        yield 2, _case(MIXTRAL, act, tokens=5, experts=4, hidden=2048, intermediate=2048)
+        yield 4, _case(DEEPSEEK, act, tokens=9, experts=8, hidden=2048, intermediate=4096)
+
+
+@pytest.mark.parametrize("parts,case", list(_part_cases()), ids=lambda v: _id(v) if isinstance(v, C.Case) else f"ks{v}")
+def test_small_units_with_k_parts(parts, case):
+    assert down_parts(case) == parts and bench._parts(case) > 1
+    _check(case)
 
 
 def test_small_kernel_is_one_launch():
