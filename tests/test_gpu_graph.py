@@ -46,10 +46,15 @@ def _fp8_cases():
             C.development(C.case("moe-fp8-mixtral-t16"), hidden=4096, intermediate=512, tokens=40),  # split gate/up
             C.development(C.BLOCK_CASES[0]),
             C.development(C.case(C.HEADLINE), tokens=8),  # the dense schedule with a shared expert
-            C.development(C.case(C.HEADLINE + "-w8a16"))]  # the W8A16 form
+            C.development(C.case(C.HEADLINE + "-w8a16")),  # the W8A16 form
+            # The decode units' form over routed lists (64 tokens of the development geometry are the
+            # batch form's), and the small form, over routed lists and in the dense schedule.
+            C.development(C.case(C.HEADLINE), tokens=40), C.development(C.case(C.HEADLINE + "-w8a16"), tokens=40),
+            C.development(C.case(C.HEADLINE), tokens=2, experts=64),
+            C.development(C.case("moe-fp8-mixtral-t16"), tokens=5, hidden=2304)]
 
 
-@pytest.mark.parametrize("case", _fp8_cases(), ids=lambda c: c.id)
+@pytest.mark.parametrize("case", _fp8_cases(), ids=lambda c: f"{c.id}-t{c.tokens}-e{c.experts}")
 def test_captured_layer_replays_equal_eager_calls(case):
     _log(f"graph capture {case.id} T={case.tokens} E={case.experts}")
     captured = submission.MoELayer(case)

@@ -117,8 +117,8 @@ def _kernels_of(call):
 def test_rows_do_not_depend_on_the_kernel_mode():
     """A row's result depends only on the row and its expert: the same 8 tokens give the same
     bits in a call of 8 tokens (decode units, 16 rows per expert at most) and as the first 8
-    of 200 tokens (100 rows per expert on average: batch units, chunks of 64 rows, the
-    per-XCD queues). I = 4096 so both calls split the down units into 8 K parts of 2 stages
+    of 200 tokens (100 rows per expert on average: batch units, chunks of up to 128 rows,
+    the per-XCD queues). I = 4096 so both calls split the down units into 8 K parts of 2 stages
     (batch mode needs an even stage count per part)."""
     base = C.case(MXCASE)
     small = C.development(base, tokens=8, experts=4, topk=2, hidden=512, intermediate=4096)

@@ -11,10 +11,12 @@ GPU tests, which call the same default path (submission.build)."""
 from __future__ import annotations
 
 import sys
+from dataclasses import replace
 
 import pytest
 import torch
 
+import bench
 from test_gpu_layer import dense_cases
 from vibe_megakernel_amd import cases as C
 from vibe_megakernel_amd import submission, workloads
@@ -134,3 +136,57 @@ def test_router_units_left_by_their_workgroups_are_rescued(monkeypatch, cid):
             torch.cuda.synchronize()
             _same(a, b, f"{case.id} with forced rescue")
         assert not one.gave_up(torch.device(DEV))
+
+
+def _form_cases():
+    """(kernel, case): every form of the single launch, both activation forms."""
+    mixtral, headline = C.case("moe-fp8-mixtral-t16"), C.case(C.HEADLINE)
+    for act in ("fp8", "bf16"):
+        a = "true" if act == "bf16" else "false"
+        form = lambda c: replace(c, activations=act)  # noqa: E731
+        yield f"k_layer<false, {a}>", form(C.development(headline, tokens=40))
+        yield f"k_layer<false, {a}>", form(C.development(mixtral, tokens=4))  # the dense schedule
+        yield f"k_layer_batch<{a}>", form(C.development(headline, tokens=90))
+        yield f"k_layer_small<{a}>", form(C.development(headline, tokens=2, experts=64))
+        yield f"k_layer_small<{a}>", form(C.development(mixtral, tokens=5, hidden=2304))  # dense
+    yield "k_layer<true, false>", C.development(mixtral, hidden=4096, intermediate=512, tokens=40)
+
+
+@pytest.mark.parametrize("kernel,case", list(_form_cases()), ids=lambda v: v if isinstance(v, str) else f"t{v.tokens}")
+def test_every_form_recovers_from_a_wait_that_gave_up(monkeypatch, kernel, case):
+    """As above, for each form's own counters (the batch form's expert counts, the small form's block
+    counters in the dense schedule), and on other inputs after it."""
+    assert bench.layer_kernel(case) == kernel
+    _log(f"give-up {kernel} T={case.tokens} E={case.experts}")
+    layer, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
+    values = _to(workloads.make_inputs(case, 8, "cpu"))
+    other = _to(workloads.make_inputs(case, 9, "cpu"))
+    layer(values)
+    monkeypatch.setenv("MEGAMOE_FORCE_WAIT_TIMEOUT", "1")
+    bad = layer(values)
+    torch.cuda.synchronize()
+    assert torch.isnan(bad["y"].float()).all() and layer.gave_up(torch.device(DEV))
+    monkeypatch.delenv("MEGAMOE_FORCE_WAIT_TIMEOUT")
+    for v in (other, values):
+        again, want = layer(v), five(v)
+        torch.cuda.synchronize()
+        _same(again, want, f"{kernel} after a forced give-up")
+        assert not layer.gave_up(torch.device(DEV))
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+def test_router_units_of_the_batch_form_are_rescued(monkeypatch, act):
+    """The same hook in the batch form, whose routing units hold four tokens: 256 router units, every odd
+    one left to them."""
+    monkeypatch.setenv("MEGAMOE_FORCE_RESCUE", "1")
+    case = replace(C.development(C.case("moe-fp8-qwen3-30b-a3b-t32"), tokens=256, hidden=2048, experts=128, topk=8),
+                   activations=act)
+    assert bench.layer_kernel(case).startswith("k_layer_batch")
+    _log(f"forced rescue {case.id} {act} T={case.tokens} E={case.experts}")
+    one, five = submission.MoELayer(case), submission.MoELayer(case, single_launch=False)
+    for seed in (11, 12):
+        values = workloads.make_inputs(case, seed, DEV)
+        a, b = one(values), five(values)
+        torch.cuda.synchronize()
+        _same(a, b, f"{case.id} with forced rescue")
+    assert not one.gave_up(torch.device(DEV))
