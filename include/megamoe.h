@@ -127,9 +127,10 @@ int megamoe_forward(const megamoe_desc* desc, const megamoe_tensors* t, void* st
  * so the call allocates nothing, in the library or in any routine it calls. For callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). No reference counterpart. t->workspace and t->workspace_bytes are
- * ignored. Returns MEGAMOE_ERR_SCRATCH, launching nothing, when megamoe_workspace_bytes(desc)
- * exceeds MEGAMOE_SCRATCH_BYTES (each of the five benchmark configs fits: Kimi-K2 at 128 tokens needs
- * 29 MiB). All calls on one GPU share its scratch: calls that overlap on that GPU (on two
+ * ignored. Returns MEGAMOE_ERR_SCRATCH, launching nothing, when the stream-ordered form needs
+ * more than MEGAMOE_SCRATCH_BYTES: at most megamoe_workspace_bytes(desc), which also holds
+ * the single launch's counters and lists (each of the five benchmark configs fits: Kimi-K2 at
+ * 128 tokens needs 31 MiB). All calls on one GPU share its scratch: calls that overlap on that GPU (on two
  * streams, or from two threads) race and must be ordered by the caller. */
 int megamoe_forward_noalloc(const megamoe_desc* desc, const megamoe_tensors* t, void* stream);
 

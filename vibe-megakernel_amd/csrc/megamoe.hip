@@ -471,7 +471,9 @@ __device__ __forceinline__ void router_tile(const uint16_t* __restrict__ x, cons
     for (int i = 0; i < NTT; ++i) acc[i] = f64x4{0.0, 0.0, 0.0, 0.0};
     // DEPTH steps of loads, and their products; steps past the end repeat the last one's loads and
     // contribute zero. PIPE (slices of several rounds, at the batch sizes): half the steps at a
-    // time, each half requested again for the next round while the other is multiplied.
+    // time, each half requested again for the next round while the other is multiplied. Macros, not
+    // lambdas: as lambdas, forced inline, the same statements took the single-launch kernels from 254
+    // VGPRs to 256 and a spill.
     constexpr int kSteps = PIPE ? kRouterDepth / 2 : kRouterDepth;
     float4 a[PIPE ? 2 : 1][kSteps];
     uint2 b[PIPE ? 2 : 1][kSteps][NTT];
@@ -995,8 +997,8 @@ __device__ __forceinline__ void select_token(const double* __restrict__ partial,
   for (int r = 0; r < NB; ++r) bias_e[r] = bias ? bias[min((int)threadIdx.x + 256 * r, E - 1)] : 0.0f;
 
   // Logits of the workgroup's tokens into LDS: thread i sums the splits (in split order)
-  // of entries i, i+256, ... (ST * E <= 64 * VPL of them, up to kMaxSplits
-  // splits each), every load issued before the first add.
+  // of entries i, i+256, ... (ST * E <= ST * 64 * VPL of them, up to kMaxSplits splits each), the
+  // loads of a round of entries issued before the round's first add.
   const int n_here = min(ST, T - t0) * E;
   if (logits_in) {
 #pragma unroll
@@ -5616,7 +5618,10 @@ size_t max_chunks(const megamoe_desc& d, int copies, int chunk = kChunkRows) {
 // least 1 / 4 / 8 blocks: one and two tokens of DeepSeek-V3's shape 122 / 108 / 106 and 148 / 149 /
 // 139 us, of Qwen3-30B-A3B's 47 / 43 / 42 and 57 / 51 / 52, of GLM-5.3-Flash's 91 / 81 / 81 and 109 /
 // 108 / 105; four of Tiny's 28 / 24 / 24; 16 at least cost Mixtral's at 1 / 2 / 4 tokens 97 -> 105,
-// 143 -> 148, 200 -> 216.
+// 143 -> 148, 200 -> 216. At 17 to 512 tokens of 8 to 32 experts, least 1 -> 8: 8 of H 2048, I 1024 at 17 /
+// 512 60 -> 45, 126 -> 96 us, 8 of H 7168, I 2048 126 -> 103, 552 -> 378. Where 8 leaves parts of 14 blocks
+// and not 7 (8 of H 4096, I 3584) neither wins throughout: 17 / 64 / 512 tokens 96 / 122 / 415 in parts of 7,
+// 98 / 121 / 407 in parts of 14, W8A16 94 / 101 / 253 and 101 / 108 / 243.
 // Depends on the geometry only, so the numerics do not depend on the device.
 constexpr size_t kDownPartBlocks = 8;
 int down_splits(const megamoe_desc& d) {
