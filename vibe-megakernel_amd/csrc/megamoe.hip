@@ -2582,7 +2582,7 @@ __device__ __forceinline__ void gateup_unit16(const GateUpArgs& a, const uint8_t
 // single launch's dense schedule), after the unit's first weight stages are requested.
 // In the dense schedule, `known`: the routing is known (the unit works its expert's routed
 // rows; else every token).
-template <bool A16 = false>
+template <bool A16>
 __device__ __forceinline__ void gateup_work(const GateUpArgs& a, int u, float (*red)[64], uint8_t* ring,
                                             const ReadyWait& ready = ReadyWait{nullptr, 0, nullptr},
                                             bool known = true) {
@@ -2590,8 +2590,7 @@ __device__ __forceinline__ void gateup_work(const GateUpArgs& a, int u, float (*
   const int4 ch = a.dense ? dense_gu_chunk(u / nbI, a.E, a.S, a.T, nbI) : a.chunks[u / nbI];
   const int j = u % nbI, jb = ch.w + j;
   // Concurrent units start at different K blocks: by unit, or by weight block where the single
-  // launch works the geometry in batch units, which do so (by block there too, GLM-5.3-Flash's shape at
-  // 37 tokens takes 422.4 us instead of 420.8).
+  // launch works the geometry in batch units, which do so.
   const int rot = (a.parts ? u : ch.x * nbI + jb) % nkb;
   const uint8_t *wg, *wu;
   const float *sg, *su;
@@ -3183,7 +3182,9 @@ __device__ __forceinline__ void down_unit(const DownArgs& a, const uint8_t* wd, 
 // matrix and K part kp (v % (nbH*ks) = j*ks + kp).
 // In the dense schedule, `known`: the routing is known (the unit works its expert's routed
 // rows; else every token).
-template <bool CO, bool A16 = false>
+// KEYED: the kernel may run a geometry of the batch form. The small form's do not, and the field read
+// for nothing cost its single launch 20 spilled SGPRs (W8A16, DeepSeek-V3's shape, one token 106.0 -> 107.2 us).
+template <bool CO, bool A16, bool KEYED>
 __device__ __forceinline__ void down_work(const DownArgs& a, int v, const ReadyWait& ready, uint8_t* ring,
                                           bool known = true) {
   const int nbH = a.H / kBlock, nbI = a.I / kBlock;
@@ -3191,7 +3192,7 @@ __device__ __forceinline__ void down_work(const DownArgs& a, int v, const ReadyW
   const int4 ch = a.dense ? dense_dn_chunk(c, a.E, a.S, a.T) : a.chunks[c];
   const int rem = v % (nbH * a.ks), j = rem / a.ks, kp = rem % a.ks;
   // Concurrent units start at different K blocks, keyed as gateup_work's.
-  const int rot = a.keyed ? down_rotation(ch.x, j >> 1, kp, a.H, a.I, a.ks) : v % (nbI / a.ks);
+  const int rot = KEYED && a.keyed ? down_rotation(ch.x, j >> 1, kp, a.H, a.I, a.ks) : v % (nbI / a.ks);
   float* pd_s = a.p_s + (size_t)kp * a.T * a.H;
   float* pd_r = a.p_r + (size_t)kp * a.rows_r * a.H;
   if (ch.x == a.E) {
@@ -3595,7 +3596,7 @@ __device__ __forceinline__ void experts_body(const ExpertArgs& args) {
       if (!(dense && e >= 0 && a.gu.offsets[e + 1] == a.gu.offsets[e])) {
         const int need = (SMALL && A16 ? per : 1) *
                          (dense ? dense_dn_need(c, a.dn.S, nbI) : (a.dn.chunks[c].x == a.dn.E ? a.dn.S * nbI : nbI));
-        down_work<false, A16>(a.dn, v,
+        down_work<false, A16, !SMALL>(a.dn, v,
                               claiming(ReadyWait{&a.ready[(size_t)c * a.ready_stride], need, &meta[kMetaError]},
                                        &meta[kMetaQueueGU], &ticket),
                               ring);
@@ -4133,7 +4134,7 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
         if constexpr (BATCH)
           down_batch_work<A16>(a.dn, v, ready, rings);
         else
-          down_work<true, A16>(a.dn, v, ready, ring, st == 1);
+          down_work<true, A16, !SMALL>(a.dn, v, ready, ring, st == 1);
       }
       ++my_down;
     }
@@ -5998,7 +5999,7 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   ga.swiglu = epi ? epi->swiglu : 0;
   ga.limit = epi ? epi->swiglu_limit : 0.0f;
   ga.dense = L.dense;
-  ga.parts = L.parts == 1 && batch_units(d) ? 0 : L.parts;
+  ga.parts = L.parts;
   ga.x16 = nullptr;  // set by the W8A16 form
   ga.h16_r = (uint16_t*)(ws + L.h16_r);
   ga.h16_s = (uint16_t*)(ws + L.h16_s);
@@ -6015,7 +6016,7 @@ void fill_expert_args(const megamoe_desc& d, const Layout& L, const megamoe_tens
   da.T = T; da.H = H; da.I = I; da.K = K; da.S = S; da.E = E;
   da.dense = L.dense;
   da.rows_r = L.rows_r;
-  da.keyed = batch_units(d) ? 1 : 0;
+  da.keyed = 0;
   da.h16_r = ga.h16_r;
   da.h16_s = ga.h16_s;
   ea.dn_of_gu = po.dn_of_gu;
@@ -6086,11 +6087,14 @@ int forward_impl(const megamoe_desc* desc, const megamoe_tensors* t, hipStream_t
   ExpertArgs ea;
   fill_expert_args(d, L, t, ws, po, epi, ea);
   if (a16) ea.gu.x16 = (const uint16_t*)x;
-  const GateUpArgs& ga = ea.gu;
   const DownArgs& da = ea.dn;
+  const bool split = !a16 && L.split;
+  if (!split && batch_units(d)) {  // the single launch runs k_layer_batch: its K rotations
+    ea.gu.parts = 0;
+    ea.dn.keyed = 1;
+  }
   // As many workgroups as fit on the device at once, and no more than the most units the
   // routing can produce.
-  const bool split = !a16 && L.split;
   const int parts = L.parts;
   const size_t units_max = expert_units_max(d, L, split ? 2 : parts, chunk);
   const size_t resident = (size_t)di.cus * di.experts_per_cu;
