@@ -2840,7 +2840,8 @@ __device__ __forceinline__ bool gateup_small_work(const GateUpArgs& a, int u, f3
     op.sx[0] = a.xs + (size_t)tok * nkb + kp * nkp;
   }
   f32x4 acc[2][1];
-  stream_gemm<2, 1, 2, 4, A16>(op, nkp, (ch.x * nbI + jb + pt) % nkp, ring, acc, ready);
+  // Two units a block (whole K): the K block that the whole-block unit starts at, so a row's sums are its.
+  stream_gemm<2, 1, 2, 4, A16>(op, nkp, (KP == 1 ? b : ch.x * nbI + jb + pt) % nkp, ring, acc, ready);
   if (KP > 1) {
     if (kp > 0) {
       part[pr * (KP - 1) + kp - 1][0][lane] = acc[0][0];
