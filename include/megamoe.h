@@ -254,7 +254,8 @@ int megamoe_layer_forward(const megamoe_desc* desc, const megamoe_tensors* t, co
  * that copies one word). No reference counterpart: the reference's eager layer has no
  * waits. Test hook: with the environment variable MEGAMOE_FORCE_WAIT_TIMEOUT=1,
  * megamoe_layer_forward's combine units wait for a count the down units never reach, for
- * 20 us, so the call reports a wait that gave up. */
+ * 20 us, so the call reports a wait that gave up; =2: odd workgroups of the batch form give up
+ * their wait for the work lists as well, while the even ones have them. */
 int megamoe_layer_status(const megamoe_desc* desc, const void* workspace, size_t workspace_bytes, int32_t* gave_up,
                          void* stream);
 

@@ -175,6 +175,34 @@ def test_every_form_recovers_from_a_wait_that_gave_up(monkeypatch, kernel, case)
 
 
 @pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("tokens", [90, 300])
+def test_batch_workgroups_that_disagree_on_the_lists_leave_no_stale_row(monkeypatch, act, tokens):
+    """The batch form's combine gives each workgroup places of its own, counted from the end of the
+    lists that it saw. The test hook makes odd workgroups give the lists up while even ones have them: all of
+    y, whose memory holds finite values before, is NaN, and the next call is whole."""
+    case = replace(C.development(C.case("moe-fp8-qwen3-30b-a3b-t32"), tokens=tokens, hidden=2048, experts=32, topk=8),
+                   activations=act)
+    assert bench.layer_kernel(case).startswith("k_layer_batch")
+    _log(f"disagreeing lists {act} T={tokens}")
+    layer = submission.MoELayer(case)
+    values = _to(workloads.make_inputs(case, 8, "cpu"))
+    good = layer(values)["y"].clone()
+    torch.cuda.synchronize()
+    monkeypatch.setenv("MEGAMOE_FORCE_WAIT_TIMEOUT", "2")
+    held = torch.full_like(good, 7.0)  # the memory that the call's y is allocated in
+    at = held.data_ptr()
+    del held
+    bad = layer(values)["y"]
+    torch.cuda.synchronize()
+    assert bad.data_ptr() == at and layer.gave_up(torch.device(DEV))
+    assert torch.isnan(bad.float()).all()
+    monkeypatch.delenv("MEGAMOE_FORCE_WAIT_TIMEOUT")
+    again = layer(values)["y"]
+    torch.cuda.synchronize()
+    assert torch.equal(again, good) and not layer.gave_up(torch.device(DEV))
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
 def test_router_units_of_the_batch_form_are_rescued(monkeypatch, act):
     """The same hook in the batch form, whose routing units hold four tokens: 256 router units, every odd
     one left to them."""

@@ -3693,7 +3693,8 @@ struct LayerArgs {
   int T, H, E, K, S, G, TG, gate, renorm, pow2;
   int nsplit, n_et, ntt, vpl, ks;
   int n_norm, n_router;
-  int force_timeout;  // test hook: the combine units wait for a flag value never raised, 20 us at most
+  int force_timeout;  // test hook, 1: the combine units wait for a flag value never raised, 20 us at most;
+                      // 2: odd workgroups of the batch form give the lists up as well
   int n_first;        // router units [0, n_first) go to the workgroup of the same index (0: none)
   int force_rescue;   // test hook: odd workgroups leave their router unit to the routing units
   int dense;          // the dense schedule (host: dense_experts); ex.ready then points at counters
@@ -4061,7 +4062,12 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
       units[0] = per * (S + E) * nbI;
       units[1] = (E + (S > 0 ? 1 : 0)) * (args.H / kBlock) * args.ks;
     } else {
-      const bool lists = load_count(my_signal_flag(ctl, kSigPermuted)) != 0;
+      bool lists = load_count(my_signal_flag(ctl, kSigPermuted)) != 0;
+      if constexpr (BATCH)
+        if (args.force_timeout == 2 && (blockIdx.x & 1)) {
+          atomicExch(&ctl[kCtlError], 1);
+          lists = false;
+        }
       units[0] = lists ? per * load_count(&args.po.meta[kMetaUnitsGU]) : 0;
       units[1] = lists ? load_count(&args.po.meta[kMetaUnitsDN]) : 0;
     }
@@ -4151,6 +4157,16 @@ __device__ __forceinline__ void layer_body(const LayerArgs& args) {
 
   // Phase 4: the combine units, once every down unit is counted (no down units: the lists
   // were not written, the error word is set and the combine writes NaN).
+  if constexpr (BATCH) {
+    // The places that the workgroups take below cover y only if every one of them saw the lists: one
+    // whose wait gave up writes the whole of y.
+    if (n_dn == 0) {
+      for (int i = threadIdx.x; i < args.T * (args.H / 8); i += 256)
+        *reinterpret_cast<uint4*>(args.y + (size_t)i * 8) =
+            make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
+      u = total;
+    }
+  }
   if (u < total) {
     ArgsPtr ap = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(ap));
@@ -6192,7 +6208,7 @@ int forward_layer_impl(const megamoe_desc* desc, const megamoe_tensors* t, const
   la.n_norm = norm ? T : 0;
   la.n_router = la.n_et * la.nsplit * passes;
   const char* force = getenv("MEGAMOE_FORCE_WAIT_TIMEOUT");
-  la.force_timeout = force && force[0] == '1' ? 1 : 0;
+  la.force_timeout = force && (force[0] == '1' || force[0] == '2') ? force[0] - '0' : 0;
 
   // As many workgroups as fit on the device at once, and no more than the most units the
   // queue can hold.
