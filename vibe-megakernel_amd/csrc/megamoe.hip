@@ -2772,8 +2772,8 @@ __device__ __forceinline__ void gateup_batch_work(const GateUpArgs& a, int u, fl
 // a CU takes in ~29 KB/us however many of its workgroups ask). The four waves work 4/KP pairs of a
 // 16-row gate and a 16-row up tile, each pair over KP = P/2 parts of the K blocks, whose sums are
 // added in part order through LDS. One call of the layer, with down_splits' longer parts: DeepSeek-V3's
-// shape, one token, W8A16 block 169 -> 108 us; Qwen3-30B-A3B's, one token, 50 -> 40; Mixtral's, five
-// tokens, 235 -> 222.
+// shape, one token, W8A16 block 169 -> 109 us; Qwen3-30B-A3B's, one token, 50 -> 40; Mixtral's, five
+// tokens, 219 -> 203 (mean of six inputs, each in another place of the memory).
 //
 // W8A16: h goes out as it is, and every unit counts towards the chunk's readiness. W8A8: h goes to
 // staging rows in bf16; the unit that finishes its block last requantizes the block's rows (per
@@ -5719,7 +5719,8 @@ bool split_gate_up(const megamoe_desc& d, int parts) {
 // The rule is a least number of rows an expert, which falls as the tokens grow. One call, decode ->
 // batch, W8A8 (W8A16 in brackets):
 //   * 16 rows at any T: Mixtral's shape at 64 / 256 / 512 tokens 296 -> 274, 541 -> 386, 949 -> 641 us; 64
-//     experts of H 2048, I 1408 at 16 rows 146 -> 136 (156 -> 138), at 15 equal.
+//     experts of H 2048, I 1408 at 16 rows 146 -> 136 (156 -> 138), at 15 equal; Tiny's at 64 tokens equal, 42.6
+//     -> 42.9 (43.9 -> 43.8).
 //   * Experts of less than 8M weights a matrix, from 208 tokens 12 rows, or 3 up to 64 experts, from 512
 //     tokens 8: Qwen3-30B-A3B's shape (128 experts) at 208 / 256 / 512 / 2000 tokens 162 -> 161, 178 -> 167,
 //     228 -> 191, 617 -> 378, with top-4 at 8 / 12.5 / 16 rows 156 -> 164, 174 -> 168, 191 -> 174, with
